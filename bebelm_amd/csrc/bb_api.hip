@@ -493,17 +493,35 @@ MoeWs moe_forward_dev(bb_ctx* c, bb_moe* m, const float* x, size_t T, float* out
   return w;
 }
 
+// Q8 buffers of one projection input (T rows of n_in), carved like the other workspaces
+// (tiled: whole tiles of 16 rows, no sums).
+bb::Q8Bufs carve_q8(Carve& cv, size_t T, size_t n_in, bool tiled) {
+  const size_t rows = tiled ? round_up(T, 16) : T;
+  int8_t* q = cv.take<int8_t>(rows * n_in);
+  float* scales = cv.take<float>(rows * n_in / 256);
+  return {q, scales, cv.take<int32_t>(tiled ? 0 : T * n_in / 32), tiled};
+}
+
+// Whether the Q8 of T rows going into these projections is tiled: every one of them that reads it
+// (Q4_K / Q6_K weights) runs on k_proj. Else it is row-major, for the row kernels.
+bool quantised(const bb_tensor* w) { return w->dtype == BB_Q4_K || w->dtype == BB_Q6_K; }
+bool tiled_input(const bb_dense* d, size_t T) {
+  return bb::proj_applies(d->gu, T, d->H) && bb::proj_applies(d->dn, T, d->F);
+}
+
 // ---- dense FFN on device pointers (model.rs:459-469 / :262-278) --------------------------------
-// xq_in (may be null): x's Q8, already computed (the decoder's fused residual + rmsnorm).
+// xq_in (may be null): x's Q8, already computed (the decoder's fused residual + rmsnorm) in the
+// layout tiled_input asks for.
 void dense_forward_dev(bb_ctx* c, bb_dense* d, const float* x, size_t T, float* out, const bb::Q8Bufs* xq_in = nullptr) {
   const size_t H = d->H, F = d->F;
+  const bool tiled = tiled_input(d, T);
   uint8_t* base = nullptr;
   for (int pass = 0; pass < 2; ++pass) {
     Carve cv{base};
-    bb::Q8Bufs xq{cv.take<int8_t>(T * H), cv.take<float>(T * H / 256), cv.take<int32_t>(T * H / 32)};
+    bb::Q8Bufs xq = carve_q8(cv, T, H, tiled);
     float* gate = cv.take<float>(T * F);
-    float* up = cv.take<float>(T * F);
-    bb::Q8Bufs aq{cv.take<int8_t>(T * F), cv.take<float>(T * F / 256), cv.take<int32_t>(T * F / 32)};
+    float* up = cv.take<float>(tiled ? 0 : T * F);
+    bb::Q8Bufs aq = carve_q8(cv, T, F, tiled);
     int32_t* grp = cv.take<int32_t>(T + 8);
     if (pass == 0) {
       base = ensure_ws(c, cv.off);
@@ -512,9 +530,18 @@ void dense_forward_dev(bb_ctx* c, bb_dense* d, const float* x, size_t T, float* 
     const int nz = T == 1;  // n_tokens == 1 takes matvec (-0.0-started sum), else matmul
     if (xq_in) xq = *xq_in;
     else launch(c, bb::K_QUANT, [&] { return bb::launch_quantize(c->stream, x, T, H, xq); });
+    if (tiled) {
+      // a batch: gate, up and swiglu, then down (matmul's sums from +0.0, the same per-(row, token)
+      // values as the row kernels)
+      launch(c, bb::K_GEMM_GATEUP,
+             [&] { return bb::launch_proj(c->stream, d->gu, true, (int)T, (int)H, (int)F, xq, gate); });
+      launch(c, bb::K_QUANT, [&] { return bb::launch_quantize(c->stream, gate, T, F, aq); });
+      launch(c, bb::K_GEMM_DOWN,
+             [&] { return bb::launch_proj(c->stream, d->dn, false, (int)T, (int)F, (int)H, aq, out); });
+      continue;
+    }
     if (T >= bb::PROJ_GEMM_MIN_T && d->gu.w && d->dn.w) {
-      // a batch: gate, up and swiglu, then down, as grouped GEMMs of one group (matmul's sums
-      // from +0.0, the same per-(row, token) values as the row kernels)
+      // a larger batch: the same as grouped GEMMs of one group
       const bb::RouteBufs rb = one_group(c, grp, T);
       launch(c, bb::K_GEMM_GATEUP, [&] {
         return bb::launch_gemm_gateup(c->stream, d->gu.dt, d->gu.w, d->gu.stride, (int)T, (int)H, (int)F, 1, 1, rb,
@@ -630,29 +657,27 @@ void matmul_dev(bb_ctx* c, uint32_t dtype, const bb_tensor* w, size_t byte_off, 
 }
 
 // ---- decoder-layer operators (bb_ops.hip) ----------------------------------------------------
-// Q8 buffers of one projection input (T rows of n_in), carved like the other workspaces.
-bb::Q8Bufs carve_q8(Carve& cv, size_t T, size_t n_in) {
-  return {cv.take<int8_t>(T * n_in), cv.take<float>(T * n_in / 256), cv.take<int32_t>(T * n_in / 32)};
-}
-
 // y = W·x for T token-major rows as the reference's operators call it: matvec1 for one token
-// (model.rs:557-560), matmul1 for a batch (:372-375); both are the row kernels (the one-token
-// form sums from -0.0 as matvec does). q: Q8 buffers for x when W is Q4_K / Q6_K.
-// With a packed form and a one-group route (rb non-null: batches of PROJ_GEMM_MIN_T tokens and
-// more) the batch runs on the grouped GEMM instead.
-// q_ready: q already holds x's Q8 (quants, scales and sums), so no quantisation is launched.
+// (model.rs:557-560), matmul1 for a batch (:372-375). q: Q8 buffers for x when W is Q4_K / Q6_K;
+// tiled, the batch runs on k_proj; else, with a packed form and a one-group route (rb non-null), on
+// the grouped GEMM, and otherwise on the row kernels (the one-token form sums from -0.0 as matvec
+// does).
+// q_ready: q already holds x's Q8, so no quantisation is launched.
 void project_dev(bb_ctx* c, const bb_tensor* w, const bb::PackedW& pk, const bb::RouteBufs* rb, size_t n_in,
                  size_t n_out, const float* x, size_t T, float* y, bb::Q8Bufs q, bool q_ready = false) {
   size_t row_bytes;
   check_weight_range(w, w->dtype, 0, n_in, n_out, row_bytes);
-  if (pk.w && rb) {
-    if (!q_ready)
-      launch(c, bb::K_QUANT, [&] { return bb::launch_quant_rows(c->stream, x, T, (int)n_in, q.q, q.scales); });
-    packed_project(c, pk, n_in, n_out, T, q, *rb, y);
-    return;
-  }
-  if (w->dtype == BB_Q4_K || w->dtype == BB_Q6_K) {
+  if (quantised(w)) {
     if (!q_ready) launch(c, bb::K_QUANT, [&] { return bb::launch_quantize(c->stream, x, T, n_in, q); });
+    if (q.tiled) {
+      launch(c, bb::K_GEMM_DOWN,
+             [&] { return bb::launch_proj(c->stream, pk, false, (int)T, (int)n_in, (int)n_out, q, y); });
+      return;
+    }
+    if (pk.w && rb) {
+      packed_project(c, pk, n_in, n_out, T, q, *rb, y);
+      return;
+    }
     launch(c, bb::K_ROWS_Q8, [&] {
       return bb::launch_rows_q8(c->stream, (int)w->dtype, w->dev, row_bytes, (int)(n_in / 256), n_out, q, n_in, T, y,
                                 n_out, T == 1);
@@ -841,28 +866,39 @@ void bb::model_adopt(bb_model* m, bb::ModelOwned&& o) { m->owned = std::move(o);
 
 namespace {
 
+bool tiled_input(const bb_conv_op* op, size_t T) {
+  return bb::proj_applies(op->in_p, T, op->H);
+}
+bool tiled_input(const bb_attn_op* op, size_t T) {
+  const size_t H = op->H;
+  return (!quantised(op->q) || bb::proj_applies(op->q_p, T, H)) && (!quantised(op->k) || bb::proj_applies(op->k_p, T, H)) &&
+         (!quantised(op->v) || bb::proj_applies(op->v_p, T, H)) && T >= bb::PROJ_MIN_T;
+}
+
 // model.rs:399-427 (T == 1) and :190-216 (T > 1) on device pointers; state [(L-1)][H] is updated.
+// xq_in (may be null): x's Q8 in the layout tiled_input asks for.
 void conv_forward_dev(bb_ctx* c, bb_conv_op* op, float* state, const float* x, size_t T, float* out,
                       const bb::Q8Bufs* xq_in = nullptr) {
   const size_t H = op->H;
   uint8_t* base = nullptr;
   for (int pass = 0; pass < 2; ++pass) {
     Carve cv{base};
-    bb::Q8Bufs xq = carve_q8(cv, T, H);
+    const bool tin = tiled_input(op, T), tout = bb::proj_applies(op->out_p, T, H);
+    bb::Q8Bufs xq = carve_q8(cv, T, H, tin);
     float* bcx = cv.take<float>(T * 3 * H);
     float* y = cv.take<float>(T * H);
-    bb::Q8Bufs yq = carve_q8(cv, T, H);
+    bb::Q8Bufs yq = carve_q8(cv, T, H, tout);
     int32_t* grp = cv.take<int32_t>(T + 8);
     if (pass == 0) {
       base = ensure_ws(c, cv.off);
       continue;
     }
     bb::RouteBufs rb{};
-    const bool gemm = T >= bb::PROJ_GEMM_MIN_T && (op->in_p.w || op->out_p.w);
+    const bool gemm = T >= bb::PROJ_GEMM_MIN_T && ((op->in_p.w && !tin) || (op->out_p.w && !tout));
     if (gemm) rb = one_group(c, grp, T);
-    project_dev(c, op->in_proj, op->in_p, gemm ? &rb : nullptr, H, 3 * H, x, T, bcx, xq_in ? *xq_in : xq,
-                xq_in != nullptr);
-    if (T == 1 && H % 256 == 0 && (op->out_proj->dtype == BB_Q4_K || op->out_proj->dtype == BB_Q6_K)) {
+    const bb::RouteBufs* rbp = gemm ? &rb : nullptr;
+    project_dev(c, op->in_proj, op->in_p, rbp, H, 3 * H, x, T, bcx, xq_in ? *xq_in : xq, xq_in != nullptr);
+    if (T == 1 && H % 256 == 0 && quantised(op->out_proj)) {
       // one token: conv, state update and y's Q8 in one launch
       launch(c, bb::K_CONV, [&] { return bb::launch_conv1_q8(c->stream, bcx, state, op->conv_w, (int)H, op->L, y, yq); });
       project_dev(c, op->out_proj, op->out_p, nullptr, H, H, y, T, out, yq, true);
@@ -870,7 +906,7 @@ void conv_forward_dev(bb_ctx* c, bb_conv_op* op, float* state, const float* x, s
     }
     launch(c, bb::K_CONV, [&] { return bb::launch_conv(c->stream, true, bcx, state, op->conv_w, (int)H, op->L, (int)T, y); });
     launch(c, bb::K_CONV_STATE, [&] { return bb::launch_conv_state(c->stream, true, bcx, state, (int)H, op->L, (int)T); });
-    project_dev(c, op->out_proj, op->out_p, gemm ? &rb : nullptr, H, H, y, T, out, yq);
+    project_dev(c, op->out_proj, op->out_p, rbp, H, H, y, T, out, yq);
   }
 }
 
@@ -902,11 +938,12 @@ void attn_forward_dev(bb_ctx* c, bb_attn_op* op, bb_kv_cache* kv, size_t pos0, c
   uint8_t* base = nullptr;
   for (int pass = 0; pass < 2; ++pass) {
     Carve cv{base};
-    bb::Q8Bufs xq = carve_q8(cv, T, H);
+    const bool tin = tiled_input(op, T), tout = bb::proj_applies(op->o_p, T, QD);
+    bb::Q8Bufs xq = carve_q8(cv, T, H, tin);
     float* q = cv.take<float>(T * QD);
     float* scores = cv.take<float>(T * NH * (n0 + T) + 4);  // (+ slack: launch_attn_pv reads one float past the rows)
     float* attn = cv.take<float>(T * QD);
-    bb::Q8Bufs aq = carve_q8(cv, T, QD);
+    bb::Q8Bufs aq = carve_q8(cv, T, QD, tout);
     int32_t* grp = cv.take<int32_t>(T + 8);
     if (pass == 0) {
       base = ensure_ws(c, cv.off);
@@ -915,14 +952,13 @@ void attn_forward_dev(bb_ctx* c, bb_attn_op* op, bb_kv_cache* kv, size_t pos0, c
     float* kn = kv->k + n0 * KV;
     float* vn = kv->v + n0 * KV;
     bb::RouteBufs rb{};
-    const bool gemm = T >= bb::PROJ_GEMM_MIN_T && (op->q_p.w || op->k_p.w || op->v_p.w || op->o_p.w);
+    const bool gemm = T >= bb::PROJ_GEMM_MIN_T &&
+                      (((op->q_p.w || op->k_p.w || op->v_p.w) && !tin) || (op->o_p.w && !tout));
     if (gemm) rb = one_group(c, grp, T);
     const bb::RouteBufs* rbp = gemm ? &rb : nullptr;
-    // x's Q8 (quants, scales and sums: both the row kernels and the GEMMs can read it) once for
-    // the three projections, or as given
+    // x's Q8 once for the three projections, or as given
     const bb::Q8Bufs xqv = xq_in ? *xq_in : xq;
-    if (!xq_in && (op->q->dtype == BB_Q4_K || op->q->dtype == BB_Q6_K || op->k->dtype == BB_Q4_K ||
-                   op->k->dtype == BB_Q6_K || op->v->dtype == BB_Q4_K || op->v->dtype == BB_Q6_K))
+    if (!xq_in && (quantised(op->q) || quantised(op->k) || quantised(op->v)))
       launch(c, bb::K_QUANT, [&] { return bb::launch_quantize(c->stream, x, T, H, xq); });
     project_dev(c, op->q, op->q_p, rbp, H, QD, x, T, q, xqv, true);
     project_dev(c, op->k, op->k_p, rbp, H, KV, x, T, kn, xqv, true);
@@ -1951,13 +1987,13 @@ void model_buffers(bb_ctx* c, bb_model* m, size_t T) {
     *p = nullptr;
   }
   m->cap_T = 0;
-  const size_t H = m->H;
+  const size_t H = m->H, Tt = round_up(T, 16);  // (nq may be tiled: whole tiles of 16 rows)
   m->h = static_cast<float*>(dev_alloc(T * H * 4));
   m->normed = static_cast<float*>(dev_alloc(T * H * 4));
   m->tmp = static_cast<float*>(dev_alloc(T * H * 4));
   if (H % 256 == 0) {
-    m->nq.q = static_cast<int8_t*>(dev_alloc(T * H));
-    m->nq.scales = static_cast<float*>(dev_alloc(T * H / 256 * 4));
+    m->nq.q = static_cast<int8_t*>(dev_alloc(Tt * H));
+    m->nq.scales = static_cast<float*>(dev_alloc(Tt * H / 256 * 4));
     m->nq.sums = static_cast<int32_t*>(dev_alloc(T * H / 32 * 4));
   }
   if (H % 256 == 0) {
@@ -2004,11 +2040,16 @@ void model_run_dev(bb_ctx* c, bb_model* m, bb_cache* k, const uint32_t* tokens, 
   });
   // Each layer boundary (h += sub-layer output, then the next rmsnorm) is one launch of
   // k_residual_norm, which also writes the normed rows' Q8 when the next sub-layer projects
-  // them (conv, attention, dense FFN; the MoE route quantises its input itself), or, before an
+  // them (conv, attention, dense FFN; the MoE route quantises its input itself) in the layout that
+  // it reads, or, before an
   // MoE layer of a few tokens, of k_residual_norm_route, which also takes the layer's router
   // logits and XQ records.
   const bool fused = H <= (size_t)bb::GU_H_MAX && m->nq.q;
-  auto boundary = [&](const float* gain, bool q8) {
+  auto op_tiled = [&](size_t i) {
+    return m->layers[i].conv ? tiled_input(m->layers[i].conv, T) : tiled_input(m->layers[i].attn, T);
+  };
+  auto boundary = [&](const float* gain, bool q8, bool tiled) {
+    m->nq.tiled = tiled;
     if (fused) {
       launch(c, bb::K_RESIDUAL_NORM, [&] {
         return bb::launch_residual_norm(c->stream, m->h, nullptr, nullptr, 0, m->tmp, gain, m->eps, H, T, m->normed,
@@ -2023,6 +2064,7 @@ void model_run_dev(bb_ctx* c, bb_model* m, bb_cache* k, const uint32_t* tokens, 
   };
   const bb::Q8Bufs* nq = fused ? &m->nq : nullptr;
   const size_t n_layers = m->layers.size();
+  m->nq.tiled = op_tiled(0);
   if (fused)
     launch(c, bb::K_RMSNORM, [&] {
       return bb::launch_rmsnorm_q8(c->stream, m->h, m->layers[0].attn_norm, m->eps, H, T, m->normed, m->nq);
@@ -2050,11 +2092,12 @@ void model_run_dev(bb_ctx* c, bb_model* m, bb_cache* k, const uint32_t* tokens, 
       const PreRoute pre{m->logits, m->xq};
       moe_forward_dev(c, L.moe, m->normed, T, m->tmp, nullptr, true, &pre);
     } else {
-      boundary(L.ffn_norm, L.dense != nullptr);
+      boundary(L.ffn_norm, L.dense != nullptr, L.dense && tiled_input(L.dense, T));
       if (L.moe) moe_forward_dev(c, L.moe, m->normed, T, m->tmp, nullptr);
       else dense_forward_dev(c, L.dense, m->normed, T, m->tmp, nq);
     }
-    boundary(i + 1 < n_layers ? m->layers[i + 1].attn_norm : nullptr, true);
+    const bool more = i + 1 < n_layers;
+    boundary(more ? m->layers[i + 1].attn_norm : nullptr, true, more && op_tiled(i + 1));
   }
   k->pos += T;
 }

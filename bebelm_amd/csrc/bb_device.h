@@ -135,19 +135,35 @@ __device__ __forceinline__ float wave_max(float v) {
 // ---- Q8 activation quantisation (matmul.rs:141-160), one 256-block per wave -----------------
 // Lane L holds elements 4L..4L+3 of the block. amax is an order-free max; the eight 32-wide
 // sums are exact integer sums over 8 lanes.
-__device__ __forceinline__ void wave_quantize_block(float4 v, int8_t* __restrict__ q, float* __restrict__ scale,
-                                                    int32_t* __restrict__ sums) {
+__device__ __forceinline__ uint32_t wave_quantize(float4 v, float& amax, int& sum4) {
+  const float a = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+  amax = wave_max(a);
+  const float inv = amax > 0.0f ? 127.0f / amax : 0.0f;
+  const int q0 = q8_round(v.x * inv), q1 = q8_round(v.y * inv), q2 = q8_round(v.z * inv), q3 = q8_round(v.w * inv);
+  sum4 = q0 + q1 + q2 + q3;
+  return (uint32_t)(q0 & 0xff) | ((uint32_t)(q1 & 0xff) << 8) | ((uint32_t)(q2 & 0xff) << 16) |
+         ((uint32_t)(q3 & 0xff) << 24);
+}
+// Block b of row t (nb blocks a row) into a batch's Q8: row-major with its per-32 sums, or (tiled)
+// the layout of k_proj.
+__device__ __forceinline__ void wave_quantize_block(float4 v, size_t t, size_t b, size_t nb, int8_t* __restrict__ q,
+                                                    float* __restrict__ scales, int32_t* __restrict__ sums,
+                                                    int tiled) {
   const int lane = threadIdx.x & 63;
-  float a = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
-  float amax = wave_max(a);
-  float inv = amax > 0.0f ? 127.0f / amax : 0.0f;
-  int q0 = q8_round(v.x * inv), q1 = q8_round(v.y * inv), q2 = q8_round(v.z * inv), q3 = q8_round(v.w * inv);
-  uint32_t packed = (uint32_t)(q0 & 0xff) | ((uint32_t)(q1 & 0xff) << 8) | ((uint32_t)(q2 & 0xff) << 16) |
-                    ((uint32_t)(q3 & 0xff) << 24);
-  reinterpret_cast<uint32_t*>(q)[lane] = packed;
-  int s = sum8(q0 + q1 + q2 + q3);
-  if ((lane & 7) == 0) sums[lane >> 3] = s;
-  if (lane == 0) *scale = amax / 127.0f;
+  float amax;
+  int sum4;
+  const uint32_t packed = wave_quantize(v, amax, sum4);
+  if (tiled) {
+    const size_t tile = (t >> 4) * nb + b, m = t & 15;
+    *reinterpret_cast<uint32_t*>(q + tile * (16 * QK) + 256 * (lane >> 2) + 16 * m + 4 * (lane & 3)) = packed;
+    if (lane == 0) scales[tile * 16 + m] = amax / 127.0f;
+    return;
+  }
+  const size_t blk = t * nb + b;
+  reinterpret_cast<uint32_t*>(q + blk * QK)[lane] = packed;
+  const int s = sum8(sum4);
+  if ((lane & 7) == 0) sums[blk * 8 + (lane >> 3)] = s;
+  if (lane == 0) scales[blk] = amax / 127.0f;
 }
 
 // ---- Q4_K (144 B: d, dmin f16 | scales[12] | qs[128]; dequant.rs:6-9) ---------------------

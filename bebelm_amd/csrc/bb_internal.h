@@ -61,10 +61,14 @@ struct RouteBufs {
   float* margin;      // [T]
 };
 
+// Q8 of a batch of rows. tiled 0: row-major quants and scales, and the per-32 sums. tiled 1: the
+// layout of k_proj, per tile of 16 tokens and super-block [16-byte chunk][token][16 B] (4 KB) and
+// the 16 scales; no sums, and both arrays hold whole tiles (the tokens rounded up to 16).
 struct Q8Bufs {
   int8_t* q;
   float* scales;
   int32_t* sums;
+  int tiled = 0;
 };
 
 // One launch = one kernel; names are used for the per-kernel profile table.
@@ -222,8 +226,21 @@ struct PackedW {
   size_t stride = 0;  // bytes of the packed matrix
   int dt = 0;
 };
-// Batches of at least this many tokens run a packed projection on the grouped GEMM (every token
-// a member of the one group); smaller ones take the row kernels.
+// Batches of PROJ_MIN_T to PROJ_MAX_T tokens run a packed projection on k_proj (bb_proj.hip); one
+// token, and matrices with no packed form, on the row kernels. Dense FFN (hidden 2048, ff 7168,
+// Q4_K) on the row kernels and here: 2 tokens 19.4 and 17.4 us, 16 tokens 76 and 18 us. Larger
+// batches run on the grouped GEMM, whose blocks share their operands through LDS (gate/up of
+// 7168, grouped GEMM and here: 130 tokens 62.6 and 23.4 us, 768 tokens 102 and 92 us, 1024 tokens
+// 107 and 127 us; down 52.5 and 13.1, 52.4 and 47.5, 55.3 and 59.2 us).
+constexpr size_t PROJ_MIN_T = 2, PROJ_MAX_T = 768;
+bool proj_applies(const PackedW& p, size_t T, size_t n_in);
+// out [T][n_out] = W·x, or silu(gate·x)·(up·x) for an interleaved gate/up matrix, from x's tiled Q8
+// (matmul's sums from +0.0).
+hipError_t launch_proj(hipStream_t s, const PackedW& p, bool gateup, int T, int n_in, int n_out, const Q8Bufs& x,
+                       float* out);
+// Batches past PROJ_MAX_T (and, from this many tokens, packed projections of an input that another
+// projection without a packed form reads too) run on the grouped GEMM (every token a member of the
+// one group).
 constexpr size_t PROJ_GEMM_MIN_T = 32;
 // The route of "every one of T tokens in group 0": counts[0] = T, offsets = {0, T}, perm = 0..T-1.
 hipError_t launch_one_group(hipStream_t s, int T, RouteBufs rb);

@@ -64,7 +64,7 @@ __global__ void __launch_bounds__(256) k_quantize(const float* __restrict__ x, s
   if (wi >= n_vec * nbk) return;
   const size_t v = wi / nbk, b = wi % nbk;
   const float4 val = *reinterpret_cast<const float4*>(x + v * n + b * QK + 4 * lane);
-  wave_quantize_block(val, q.q + v * n + b * QK, q.scales + v * nbk + b, q.sums + v * (n / 32) + b * 8);
+  wave_quantize_block(val, v, b, nbk, q.q, q.scales, q.sums, q.tiled);
 }
 
 hipError_t launch_quantize(hipStream_t s, const float* x, size_t n_vec, size_t n, Q8Bufs q) {
@@ -433,7 +433,7 @@ __global__ void __launch_bounds__(256) k_rmsnorm(const float* __restrict__ x, co
     const int lane = threadIdx.x & 63;
     for (size_t b = threadIdx.x >> 6; b < nbk; b += 4) {
       const float4 val = *reinterpret_cast<const float4*>(s_norm + b * QK + 4 * lane);
-      wave_quantize_block(val, q.q + v * n + b * QK, q.scales + v * nbk + b, q.sums + v * (n / 32) + b * 8);
+      wave_quantize_block(val, v, b, nbk, q.q, q.scales, q.sums, q.tiled);
     }
   } else if (regs) {
 #pragma unroll
@@ -539,7 +539,7 @@ __global__ void __launch_bounds__(256) k_residual_norm(float* __restrict__ h, co
     const int lane = threadIdx.x & 63;
     for (size_t b = threadIdx.x >> 6; b < nbk; b += 4) {
       const float4 val = *reinterpret_cast<const float4*>(s_norm + b * QK + 4 * lane);
-      wave_quantize_block(val, q.q + t * n + b * QK, q.scales + t * nbk + b, q.sums + t * (n / 32) + b * 8);
+      wave_quantize_block(val, t, b, nbk, q.q, q.scales, q.sums, q.tiled);
     }
     return;
   }

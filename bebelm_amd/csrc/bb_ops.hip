@@ -99,8 +99,7 @@ __global__ void __launch_bounds__(64) k_conv1_q8(const float* __restrict__ src, 
     for (int k = 0; k + 1 < L; ++k) state[(size_t)k * C + c] = conv_col<true>(src, state, C, L, 1 + k, c);
   }
   *reinterpret_cast<float4*>(y + c0) = make_float4(out[0], out[1], out[2], out[3]);
-  wave_quantize_block(make_float4(out[0], out[1], out[2], out[3]), q.q + blockIdx.x * QK, q.scales + blockIdx.x,
-                      q.sums + blockIdx.x * 8);
+  wave_quantize_block(make_float4(out[0], out[1], out[2], out[3]), 0, blockIdx.x, gridDim.x, q.q, q.scales, q.sums, 0);
 }
 
 hipError_t launch_conv1_q8(hipStream_t s, const float* src, float* state, const float* w, int C, int L, float* y,
