@@ -941,7 +941,7 @@ void attn_forward_dev(bb_ctx* c, bb_attn_op* op, bb_kv_cache* kv, size_t pos0, c
     const bool tin = tiled_input(op, T), tout = bb::proj_applies(op->o_p, T, QD);
     bb::Q8Bufs xq = carve_q8(cv, T, H, tin);
     float* q = cv.take<float>(T * QD);
-    float* scores = cv.take<float>(T * NH * (n0 + T) + 4);  // (+ slack: launch_attn_pv reads one float past the rows)
+    float* scores = cv.take<float>(T * NH * (size_t)bb::attn_ld((int)(n0 + T)) + 4);  // (+ slack: launch_attn_pv reads one float past the rows)
     float* attn = cv.take<float>(T * QD);
     bb::Q8Bufs aq = carve_q8(cv, T, QD, tout);
     int32_t* grp = cv.take<int32_t>(T + 8);
@@ -1676,7 +1676,7 @@ int bb_attention_decode(bb_ctx* c, const float* q, const float* k, const float* 
     with_io(c, loc, {{q, QD * 4, true, false}, {k, KVB, true, false}, {v, KVB, true, false}, {out, QD * 4, false, true}},
             [&](std::vector<void*>& d) {
               // (a float of slack after the rows: launch_attn_pv reads up to one past a row's end)
-              float* scores = reinterpret_cast<float*>(ensure_ws(c, n_heads * n_ctx * 4 + 16));
+              float* scores = reinterpret_cast<float*>(ensure_ws(c, n_heads * (size_t)bb::attn_ld((int)n_ctx) * 4 + 16));
               const int n0 = (int)n_ctx - 1;
               launch(c, bb::K_ATTN_SCORES, [&] {
                 return bb::launch_attn_scores(c->stream, static_cast<const float*>(d[0]),

@@ -298,7 +298,10 @@ hipError_t launch_conv1_q8(hipStream_t s, const float* src, float* state, const 
 hipError_t launch_norm_rope(hipStream_t s, float* buf, int T, int n_heads, int hd, const float* gain, float eps,
                             const float2* rope, float* buf2 = nullptr, int n2 = 0,
                             const float* gain2 = nullptr);
-// scores [T][n_heads][n0+T]: token t's query against cached positions j < n0 + t + 1.
+// Floats of a score row of up to n positions: whole 16-position pieces, so rows start 64-byte
+// aligned.
+constexpr int attn_ld(int n) { return (n + 15) / 16 * 16; }
+// scores [T][n_heads][attn_ld(n0+T)]: token t's query against cached positions j < n0 + t + 1.
 hipError_t launch_attn_scores(hipStream_t s, const float* q, const float* kc, int n0, int T, int n_heads, int n_kv,
                               int hd, float scale, float* scores);
 // softmax of each score row (in place), then out [T][n_heads][hd] = Σ_j w_j·v_j. scores needs one

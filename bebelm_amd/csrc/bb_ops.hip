@@ -29,6 +29,11 @@ constexpr int PV_CHUNK = 32;    // value-column loads in flight per lane in P·V
 constexpr int PVL_MIN_LD = 0;   // rows from this length take the softmax + k_attn_pv_long pair
 constexpr int AT_PV_MIN_T = 8;  // batches of this many tokens take the tiled softmax + P·V
 
+template <class F, int... I>
+__device__ __forceinline__ void unroll_seq(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
 // ---- gated short conv ------------------------------------------------------------------------
 // Column j of [state; bx] for channel c (j < L-1: the state; else token j-(L-1) of the batch).
 // OP: the batch is the in_proj output (B, C, x_gate chunks of 3C per token) and bx = B·x_gate.
@@ -244,6 +249,45 @@ __device__ __forceinline__ void row_to_lds(const float* src, float* lrow, int n)
   __builtin_amdgcn_s_waitcnt(0x3f70);  // vmcnt(0): the copies landed
 }
 
+// The reference's normaliser from a tree sum st of n exps, or false where it does not decide it (see
+// row_softmax): inv = (float)(1 / sum).
+__device__ __forceinline__ bool softmax_inv(int n, double st, float* inv) {
+  const double bnd = (double)(n + 64) * 0x1p-51 * st;
+  const float f_lo = (float)(1.0 / (st - bnd)), f_hi = (float)(1.0 / (st + bnd));
+  if (f_lo != f_hi) return false;
+  *inv = f_lo;
+  return true;
+}
+
+// The same from the chain itself, left to right; the next 16 values are read while the adds of the
+// current 16 run (the adds are one dependent chain, the reads are not). One lane.
+template <bool LDS>
+__device__ void softmax_inv_chain(const Row<LDS> r, int n, float* inv) {
+  constexpr int U = 16;
+  double sum = 0.0;
+  const int nfull = n / U;
+  float ea[U], eb[U];
+  auto rd = [&](float(&e)[U], int c) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) e[u] = r.ld(c * U + u);
+  };
+  auto add = [&](const float(&e)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) sum += (double)e[u];
+  };
+  if (nfull > 0) rd(ea, 0);
+  int c = 0;
+  for (; c + 2 <= nfull; c += 2) {
+    rd(eb, c + 1);
+    add(ea);
+    if (c + 2 < nfull) rd(ea, c + 2);
+    add(eb);
+  }
+  if (c < nfull) add(ea);
+  for (int j = nfull * U; j < n; ++j) sum += (double)r.ld(j);
+  *inv = (float)(1.0 / sum);
+}
+
 // softmax.rs:9-22 on row r[0..n) by the block's NW waves (exps written back, then scaled).
 template <bool LDS, int NW = 1>
 __device__ void row_softmax(const Row<LDS> r, int n, const uint64_t* exptab, float* s_inv) {
@@ -287,37 +331,7 @@ __device__ void row_softmax(const Row<LDS> r, int n, const uint64_t* exptab, flo
 #pragma unroll
     for (int i = 1; i < NW; ++i) st += wsum[i];
   }
-  const double bnd = (double)(n + 64) * 0x1p-51 * st;
-  const float f_lo = (float)(1.0 / (st - bnd)), f_hi = (float)(1.0 / (st + bnd));
-  if (f_lo == f_hi) {
-    if (tid == 0) *s_inv = f_lo;
-  } else if (tid == 0) {
-    // left to right; the next 16 values are read while the adds of the current 16 run (the adds
-    // are one dependent chain, the reads are not)
-    constexpr int U = 16;
-    double sum = 0.0;
-    const int nfull = n / U;
-    float ea[U], eb[U];
-    auto rd = [&](float(&e)[U], int c) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) e[u] = r.ld(c * U + u);
-    };
-    auto add = [&](const float(&e)[U]) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) sum += (double)e[u];
-    };
-    if (nfull > 0) rd(ea, 0);
-    int c = 0;
-    for (; c + 2 <= nfull; c += 2) {
-      rd(eb, c + 1);
-      add(ea);
-      if (c + 2 < nfull) rd(ea, c + 2);
-      add(eb);
-    }
-    if (c < nfull) add(ea);
-    for (int j = nfull * U; j < n; ++j) sum += (double)r.ld(j);
-    *s_inv = (float)(1.0 / sum);
-  }
+  if (tid == 0 && !softmax_inv(n, st, s_inv)) softmax_inv_chain(r, n, s_inv);
   __syncthreads();
   const float inv = *s_inv;
 #pragma unroll 8
@@ -379,8 +393,6 @@ __global__ void __launch_bounds__(64) k_attn_softmax_pv(float* sc, const float* 
 constexpr int AT_HD = 64;
 constexpr int AT_KS = AT_HD + 4;  // padded LDS row of a key (conflict-free float4 reads)
 constexpr int AT_ITEMS = 64;     // items of a scores block
-constexpr int AT_PV_ITEMS = 16;  // items of a P·V block (more blocks: its waves run long chains)
-constexpr int AT_IPW = AT_PV_ITEMS / 4;  // P·V items per wave
 
 __host__ __device__ constexpr int at_tokens(int G, int items = AT_ITEMS) { return G >= items ? 1 : items / G; }
 
@@ -472,60 +484,299 @@ __global__ void __launch_bounds__(64 * SM_WAVES) k_attn_softmax(float* sc, int n
     for (int j = tid; j < n; j += 64 * SM_WAVES) s[j] = lrow[j];
 }
 
-// out[t][h][d] = Σ_j p[t][h][j]·v[j][g][d] for the block's items, position order from 0.0. Per
-// chunk of 64 positions the value rows and the items' probabilities are copied into LDS; lane d
-// of wave w keeps the running sums of items w, w+4, ... (independent chains side by side).
-__global__ void __launch_bounds__(256) k_attn_pv_tile(const float* __restrict__ p, const float* __restrict__ vc,
-                                                      int n0, int T, int n_heads, int n_kv, int ld,
-                                                      float* __restrict__ out) {
-  __shared__ __align__(16) float sv[64 * AT_HD];
-  __shared__ __align__(16) float sp[AT_PV_ITEMS * 64];
-  const int G = n_heads / n_kv, TT = at_tokens(G, AT_PV_ITEMS);
-  const int g = blockIdx.x, t0 = blockIdx.y * TT;
-  const int nt = min(TT, T - t0), n_items = nt * G;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int jlast = n0 + t0 + nt - 1;  // the last position any item uses
-  float o[AT_IPW];
-  int lim[AT_IPW];  // item w + 4k uses positions j <= lim[k] (-1: no such item)
+// The same with the row in registers, SR_V x 4 values a thread, read and written once: rows of at
+// most 256 SR_V NW positions (16384 for the largest block). A batch's rows are then one pass over
+// memory (512 tokens x 32 heads on 4000 positions: 2 x 262 MB, 65 us instead of 112 through LDS;
+// on 512 positions 16 us instead of 53; one token on 9001 positions, with its P·V, 50 -> 47 us).
+constexpr int SR_V = 4;
+template <int NW>
+__global__ void __launch_bounds__(64 * NW) k_attn_softmax_reg(float* sc, int n0, int n_heads, int ld) {
+  __shared__ uint64_t exptab[32];
+  __shared__ float s_inv, wmax[NW];
+  __shared__ double wsum[NW];
+  const int h = blockIdx.x, t = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int n = n0 + t + 1;
+  float* const s = sc + ((size_t)t * n_heads + h) * ld;
+  const uint64_t exp_e = exp_table_entry();
+  // (rows are whole 16-position pieces: a piece that starts inside the row is inside its padding)
+  float v[SR_V][4];
 #pragma unroll
-  for (int k = 0; k < AT_IPW; ++k) {
-    const int it = w + 4 * k;
-    o[k] = 0.0f;
-    lim[k] = it < n_items ? n0 + t0 + it / G : -1;
+  for (int k = 0; k < SR_V; ++k) {
+    const int j = 4 * (tid + 64 * NW * k);
+    const float4 x = *reinterpret_cast<const float4*>(s + (j < n ? j : 0));
+    v[k][0] = x.x;
+    v[k][1] = x.y;
+    v[k][2] = x.z;
+    v[k][3] = x.w;
   }
-  for (int c0 = 0; c0 <= jlast; c0 += 64) {
-    __syncthreads();  // the previous chunk has been used
-    for (int i = tid; i < 64 * (AT_HD / 4); i += 256) {
-      const int r = i / (AT_HD / 4), c4 = i % (AT_HD / 4);
-      const int jj = min(c0 + r, jlast);
-      reinterpret_cast<float4*>(sv)[i] = reinterpret_cast<const float4*>(vc + ((size_t)jj * n_kv + g) * AT_HD)[c4];
+  if (tid < 32) exptab[tid] = exp_e;
+  float m = -__builtin_inff();
+#pragma unroll
+  for (int k = 0; k < SR_V; ++k)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (4 * (tid + 64 * NW * k) + i < n) m = fmaxf(m, v[k][i]);
+  m = wave_max(m);
+  if (lane == 0) wmax[w] = m;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NW; ++i) m = fmaxf(m, wmax[i]);
+  double st = 0.0;
+#pragma unroll
+  for (int k = 0; k < SR_V; ++k)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bool in = 4 * (tid + 64 * NW * k) + i < n;
+      v[k][i] = in ? bb_expf_tab(v[k][i] - m, exptab) : 0.0f;
+      st += (double)v[k][i];
     }
-    for (int i = tid; i < n_items * 64; i += 256) {
-      const int it = i >> 6, jj = c0 + (i & 63), t = t0 + it / G, hh = it % G;
-      sp[i] = jj <= n0 + t ? p[((size_t)t * n_heads + (size_t)g * G + hh) * ld + jj] : 0.0f;
-    }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) st += __shfl_xor(st, o);
+  if (lane == 0) wsum[w] = st;
+  __syncthreads();
+  st = wsum[0];
+#pragma unroll
+  for (int i = 1; i < NW; ++i) st += wsum[i];
+  float inv;
+  if (!softmax_inv(n, st, &inv)) {  // the same in every thread
+    const Row<false> r{s};
+#pragma unroll
+    for (int k = 0; k < SR_V; ++k)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (const int j = 4 * (tid + 64 * NW * k) + i; j < n) r.st(j, v[k][i]);
     __syncthreads();
-    const int jn = min(64, jlast - c0 + 1);
-    for (int jj = 0; jj < jn; ++jj) {
-      const float v = sv[jj * AT_HD + lane];
-      const int j = c0 + jj;
-      // branch-free: every item adds its product, with the bits cleared (+0.0) where the item
-      // does not see position j. Adding +0.0 leaves a sum unchanged: the sums start at +0.0 and
-      // never become -0.0 (x + y rounds an exact zero to +0.0), so they are the ones of adding
-      // only the positions seen.
-#pragma unroll
-      for (int k = 0; k < AT_IPW; ++k) {
-        const uint32_t keep = j <= lim[k] ? 0xffffffffu : 0u;
-        const float pv = sp[(w + 4 * k) * 64 + jj] * v;
-        o[k] += __uint_as_float(__float_as_uint(pv) & keep);
-      }
-    }
+    if (tid == 0) softmax_inv_chain(r, n, &s_inv);
+    __syncthreads();
+    inv = s_inv;
   }
 #pragma unroll
-  for (int k = 0; k < AT_IPW; ++k) {
-    const int it = w + 4 * k;
-    if (it < n_items)
-      out[((size_t)(t0 + it / G) * n_heads + (size_t)g * G + it % G) * AT_HD + lane] = o[k];
+  for (int k = 0; k < SR_V; ++k)
+    if (const int j = 4 * (tid + 64 * NW * k); j < n)
+      *reinterpret_cast<float4*>(s + j) = make_float4(v[k][0] * inv, v[k][1] * inv, v[k][2] * inv, v[k][3] * inv);
+}
+
+// ---- attention of a batch on f32 MFMA (head_dim 64) ------------------------------------------------
+// v_mfma_f32_16x16x1_4b_f32 forms 4 x (16 x 16) outer products, each element one fused
+// multiply-add with a single rounding (denormals and signs of zero included): fmaf(a, b, c). It
+// shares the SIMD's multipliers with the vector instructions (the two do not overlap), but makes
+// 1,024 of them in the time of 13 vector instructions instead of 16, and takes its operands from
+// per-lane registers, so nothing is broadcast through LDS.
+// A tile is 16 items = (token, head) pairs of one kv head, 16 / G tokens. Lane l = 16 g + r. D
+// register 4b + i of lane l is element (row 4g + i of A's block, column r of B's) of block b.
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+// Scores: A = the keys (lane = position of a chunk of 64, its row in registers), B = the items'
+// queries (lane (g, r) holds elements 16m + 4g.. of item r; blgp 4 + g broadcasts group g's to all
+// four blocks). Chain c of matmul.rs:36-66's dot is two MFMAs (elements c and c + 32), and the 32
+// chains are summed in the reference's tree on whole registers of 16 scores.
+template <int C>
+__device__ __forceinline__ v16f score_chain(const float (&k)[AT_HD], const float4 (&q)[4]) {
+  constexpr int g = (C / 4) % 4, m = C / 16, i = C % 4;
+  v16f d = __builtin_amdgcn_mfma_f32_16x16x1f32(k[C], reinterpret_cast<const float*>(&q[m])[i], v16f{}, 0, 0, 4 + g);
+  return __builtin_amdgcn_mfma_f32_16x16x1f32(k[C + 32], reinterpret_cast<const float*>(&q[m + 2])[i], d, 0, 0, 4 + g);
+}
+template <int J>
+__device__ __forceinline__ v16f score_lane(const float (&k)[AT_HD], const float4 (&q)[4]) {
+  const v16f x = score_chain<J>(k, q) + score_chain<J + 8>(k, q);
+  const v16f y = score_chain<J + 16>(k, q) + score_chain<J + 24>(k, q);
+  v16f v = x + y;
+  // formed here: chains hoisted from the lanes that follow would not fit the registers
+  asm volatile("" : "+v"(v));
+  __builtin_amdgcn_sched_barrier(0);
+  return v;
+}
+
+// Block = 64 positions of one kv head (the key rows copied into LDS once, coalesced) against
+// AT_SC_TILES item tiles, 4 waves taking them in turn. Causal: item (t, .) covers j <= n0 + t; a
+// tile none of whose tokens sees the chunk is skipped, and scores past an item's own position are
+// written but never read (rows hold whole 16-position pieces: ld). Per 1,024 scores 64 MFMAs and 496
+// adds, about 1.7 us of a SIMD; 4000 tokens in chunks of 512: 633 us, against 895 us for the form
+// whose lanes held a key and read every query element from LDS (k_attn_scores_tile, still the
+// better one for the few items of a decode step). Two waves a SIMD: a key row, the queries and up
+// to six partial sums of 16 take 256 registers.
+constexpr int AT_SC_TILES = 16;
+__global__ void __launch_bounds__(256, 2) k_attn_scores_mfma(const float* __restrict__ q, const float* __restrict__ kc,
+                                                             int n0, int T, int n_heads, int n_kv, float scale,
+                                                             float* __restrict__ sc, int ld) {
+  __shared__ __align__(16) float sk[64 * AT_KS];
+  const int G = n_heads / n_kv, TT = at_tokens(G, 16);
+  const int g0 = blockIdx.x, j0 = blockIdx.y * 64, first = blockIdx.z * AT_SC_TILES;
+  const int n_tiles = (T + TT - 1) / TT, last = min(first + AT_SC_TILES, n_tiles);
+  if (j0 > n0 + min(last * TT, T) - 1) return;  // no token of the block sees these positions
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 15, g = lane >> 4;
+  const int jlast = n0 + T - 1;  // last cached position (rows past it are clamped, never used)
+  for (int i = tid; i < 64 * (AT_HD / 4); i += 256) {
+    const int row = i / (AT_HD / 4), c4 = i % (AT_HD / 4);
+    *reinterpret_cast<float4*>(sk + row * AT_KS + 4 * c4) =
+        reinterpret_cast<const float4*>(kc + ((size_t)min(j0 + row, jlast) * n_kv + g0) * AT_HD)[c4];
+  }
+  __syncthreads();
+  float kr[AT_HD];
+#pragma unroll
+  for (int c4 = 0; c4 < AT_HD / 4; ++c4) {
+    const float4 v = *reinterpret_cast<const float4*>(sk + lane * AT_KS + 4 * c4);
+    kr[4 * c4] = v.x;
+    kr[4 * c4 + 1] = v.y;
+    kr[4 * c4 + 2] = v.z;
+    kr[4 * c4 + 3] = v.w;
+  }
+  // item r of tile `it` (past the tile's items: its last one again, not stored)
+  auto item_row = [&](int it, int& n_items) {
+    const int t0 = it * TT;
+    n_items = min(TT, T - t0) * G;
+    const int i = min(r, n_items - 1);
+    return (size_t)(t0 + i / G) * n_heads + (size_t)g0 * G + i % G;
+  };
+  for (int it = first + w; it < last; it += 4) {
+    if (j0 > n0 + min((it + 1) * TT, T) - 1) continue;  // (no barrier follows)
+    int n_items;
+    const size_t row = item_row(it, n_items);
+    const float4* qr = reinterpret_cast<const float4*>(q + row * AT_HD) + g;
+    float4 q4[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) q4[m] = qr[4 * m];
+    v16f a = score_lane<0>(kr, q4) + score_lane<4>(kr, q4);
+    v16f b = score_lane<2>(kr, q4) + score_lane<6>(kr, q4);
+    const v16f even = a + b;
+    a = score_lane<1>(kr, q4) + score_lane<5>(kr, q4);
+    b = score_lane<3>(kr, q4) + score_lane<7>(kr, q4);
+    const v16f d = even + (a + b);
+    if (r < n_items) {
+      float* o = sc + row * ld + j0 + 4 * g;
+#pragma unroll
+      for (int bl = 0; bl < 4; ++bl)
+        if (j0 + 16 * bl + 4 * g < ld)
+          *reinterpret_cast<float4*>(o + 16 * bl) =
+              make_float4(d[4 * bl] * scale, d[4 * bl + 1] * scale, d[4 * bl + 2] * scale, d[4 * bl + 3] * scale);
+    }
+  }
+}
+
+// P·V: out[t][h][d] = Σ_j p[t][h][j]·v[j][g][d] in position order from 0.0 (attention.rs:46-54: a
+// rounded multiply, then an add). One wave keeps the running sums of one item tile and 64 / S
+// dims; the four blocks of an MFMA are those 64 / S dims (16 a block) at S positions, and its exact
+// products are then added position by position: 16 adds an MFMA. (A product of -0 arrives as +0; a
+// sum that starts at +0 is never -0, so it is the same.) A lane of group g loads four probabilities
+// of item r, those of the positions that cbsz / abid hand from its group to the blocks; the value
+// rows come one dword a lane an MFMA, lane = (position, dim). Chunks of 16 positions, PV_AHEAD in
+// flight. Positions an item does not see are cleared to +0, which leaves its sum unchanged: the
+// tile's last chunks only.
+// A wave alone on its SIMD issues these adds at half the rate that two together reach, so S is
+// chosen for 2048 waves. 4000 tokens in chunks of 512 (32 heads, 8 kv heads), P·V of all chunks: 809
+// us, 24 us per 512 positions against 18 at the rates of the adds and MFMAs alone; with S = 1 (1024
+// waves a chunk) 1157 us, and 2177 us for the form before (value rows and probabilities in LDS,
+// multiplied and added lane = dim: five LDS reads per four items and position).
+constexpr int PV_AHEAD = 3;
+template <int S>
+__global__ void __launch_bounds__(256, 2) k_attn_pv_mfma(const float* __restrict__ p, const float* __restrict__ vc,
+                                                         int n0, int T, int n_heads, int n_kv, int ld,
+                                                         float* __restrict__ out) {
+  static_assert(S == 2 || S == 4, "positions an MFMA");
+  constexpr int DG = 4 / S;      // 16-dim groups of the wave
+  constexpr int NM = 16 / S;     // MFMAs a chunk: 4 for each of its NM / 4 spans of 4 S positions
+  const int G = n_heads / n_kv, TT = at_tokens(G, 16);
+  const int g0 = blockIdx.x, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int tile = blockIdx.y * (4 / S) + w / S, d0 = (w % S) * 16 * DG;
+  const int t0 = tile * TT;
+  if (t0 >= T) return;  // (a whole wave: the block has no barrier)
+  const int r = lane & 15, g = lane >> 4;
+  const int nt = min(TT, T - t0), n_items = nt * G;
+  const int i0 = min(r, n_items - 1);
+  // group g's four positions of a chunk: span g % (4 / S), quad g / (4 / S) of it
+  const float* prow = p + ((size_t)(t0 + i0 / G) * n_heads + (size_t)g0 * G + i0 % G) * ld +
+                      (g % DG) * 4 * S + (g / DG) * 4;
+  const int n_all = n0 + t0 + nt;      // positions the tile's last token sees
+  const int nfull = (n0 + t0 + 1) / 16, nch = (n_all + 15) / 16;
+  const uint32_t vrow = (uint32_t)n_kv * 256u;                // bytes of a cache row
+  const __amdgpu_buffer_rsrc_t rv = buf_rsrc(vc, (uint32_t)n_all * vrow);  // (positions past n_all read zero)
+  // lane (block b = g, column r): position quad b / DG, dim group b % DG
+  const uint32_t vl = (uint32_t)(g / DG) * 4u * vrow + (uint32_t)g0 * 256u + 4u * (uint32_t)(d0 + 16 * (g % DG) + r);
+  struct Chunk {
+    float4 p;
+    float v[NM];
+  };
+  auto load = [&](Chunk& x, int c) {
+    x.p = *reinterpret_cast<const float4*>(prow + 16 * min(c, nch - 1));
+    // (the chunk's offset in the lane's: the range check then covers it)
+    const uint32_t vo = vl + (uint32_t)(16 * min(c, nch - 1)) * vrow;
+#pragma unroll
+    for (int m = 0; m < NM; ++m) x.v[m] = buf_load4f(rv, vo + (uint32_t)((m / 4) * 4 * S + m % 4) * vrow, 0);
+  };
+  float acc[4 * DG];
+#pragma unroll
+  for (int k = 0; k < 4 * DG; ++k) acc[k] = 0.0f;
+  auto products = [&](const Chunk& x, auto SPAN, v16f (&d)[4]) {
+    constexpr int span = decltype(SPAN)::value;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      d[q] = __builtin_amdgcn_mfma_f32_16x16x1f32(reinterpret_cast<const float*>(&x.p)[q], x.v[4 * span + q], v16f{},
+                                                  S == 2 ? 1 : 0, S == 2 ? span : 0, 0);
+  };
+  auto full = [&](const Chunk& x) {
+    unroll_seq(
+        [&](auto SPAN) {
+          v16f d[4];
+          products(x, SPAN, d);
+#pragma unroll
+          for (int po = 0; po < S; ++po)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+              for (int k = 0; k < 4 * DG; ++k) acc[k] += d[q][4 * DG * po + k];
+        },
+        std::make_integer_sequence<int, NM / 4>{});
+  };
+  constexpr int NB = PV_AHEAD + 1;
+  Chunk x[NB];
+  unroll_seq(
+      [&](auto U) {
+        load(x[decltype(U)::value], decltype(U)::value);
+        __builtin_amdgcn_sched_barrier(0);
+      },
+      std::make_integer_sequence<int, PV_AHEAD>{});
+  int c = 0;
+  for (; c + NB <= nfull; c += NB) {
+    unroll_seq(
+        [&](auto U) {
+          constexpr int u = decltype(U)::value;
+          load(x[(u + PV_AHEAD) % NB], c + u + PV_AHEAD);
+          __builtin_amdgcn_sched_barrier(0);
+          full(x[u]);
+          __builtin_amdgcn_sched_barrier(0);
+        },
+        std::make_integer_sequence<int, NB>{});
+  }
+  int lim[4];  // item 4g + i sees positions up to lim[i]
+#pragma unroll
+  for (int i = 0; i < 4; ++i) lim[i] = n0 + t0 + (4 * g + i) / G;
+  for (; c < nch; ++c) {
+    unroll_seq(
+        [&](auto SPAN) {
+          v16f d[4];
+          products(x[0], SPAN, d);
+#pragma unroll
+          for (int po = 0; po < S; ++po)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const int pos = 16 * c + decltype(SPAN)::value * 4 * S + 4 * po + q;
+#pragma unroll
+              for (int k = 0; k < 4 * DG; ++k) acc[k] += pos <= lim[k % 4] ? d[q][4 * DG * po + k] : 0.0f;
+            }
+        },
+        std::make_integer_sequence<int, NM / 4>{});
+#pragma unroll
+    for (int k = 0; k + 1 < PV_AHEAD; ++k) x[k] = x[k + 1];
+    load(x[PV_AHEAD - 1], c + PV_AHEAD);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int it = 4 * g + i;
+    if (it < n_items) {
+      float* o = out + ((size_t)(t0 + it / G) * n_heads + (size_t)g0 * G + it % G) * AT_HD + d0 + r;
+#pragma unroll
+      for (int dg = 0; dg < DG; ++dg) o[16 * dg] = acc[4 * dg + i];
+    }
   }
 }
 
@@ -569,11 +820,6 @@ struct PvlCfg {
   static constexpr int D = D0 < 12 ? D0 : 12;        // chunks of loads in flight (NLD·D fits vmcnt)
   static_assert(NL * 4 * HP * NP == 64, "the producers' lanes make the chunk's 64 x 64 products");
 };
-
-template <class F, int... I>
-__device__ __forceinline__ void unroll_seq(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
 
 template <int G>
 __global__ void __launch_bounds__(320) k_attn_pv_long(const float* __restrict__ p, const float* __restrict__ vc,
@@ -766,9 +1012,20 @@ __global__ void __launch_bounds__(320) k_attn_pv_long(const float* __restrict__ 
   }
 }
 
+// A batch large enough to fill item tiles: scores and P·V on MFMA.
+static bool attn_batch(int T, int hd, int n_heads, int n_kv) {
+  return T >= AT_PV_MIN_T && hd == AT_HD && n_heads / n_kv <= 16;
+}
+
 hipError_t launch_attn_scores(hipStream_t s, const float* q, const float* kc, int n0, int T, int n_heads, int n_kv,
                               int hd, float scale, float* scores) {
-  const int ld = n0 + T;
+  const int ld = attn_ld(n0 + T);
+  if (attn_batch(T, hd, n_heads, n_kv)) {
+    const int tiles = (T + at_tokens(n_heads / n_kv, 16) - 1) / at_tokens(n_heads / n_kv, 16);
+    BB_LAUNCH(k_attn_scores_mfma, dim3(n_kv, (unsigned)((n0 + T + 63) / 64), (unsigned)((tiles + AT_SC_TILES - 1) / AT_SC_TILES)),
+              dim3(256), 0, s, q, kc, n0, T, n_heads, n_kv, scale, scores, ld);
+    return hipGetLastError();
+  }
   if (hd == AT_HD && n_heads / n_kv <= AT_ITEMS) {
     const int TT = at_tokens(n_heads / n_kv);
     BB_LAUNCH(k_attn_scores_tile, dim3((unsigned)((ld + 63) / 64), n_kv, (unsigned)((T + TT - 1) / TT)), dim3(256), 0,
@@ -784,30 +1041,45 @@ hipError_t launch_attn_scores(hipStream_t s, const float* q, const float* kc, in
   return hipGetLastError();
 }
 
+// Every row's softmax in place: in registers up to 16384 positions, past them through LDS, past
+// OPS_ROW_LDS in memory.
+static hipError_t launch_attn_softmax(hipStream_t s, float* scores, int n0, int T, int n_heads, int ld) {
+  const dim3 grid(n_heads, T);
+#define BB_SOFTMAX_REG(nw)                                                                          \
+  if (ld <= 256 * SR_V * nw) {                                                                      \
+    BB_LAUNCH(k_attn_softmax_reg<nw>, grid, dim3(64 * nw), 0, s, scores, n0, n_heads, ld);          \
+    return hipGetLastError();                                                                       \
+  }
+  BB_SOFTMAX_REG(1) BB_SOFTMAX_REG(2) BB_SOFTMAX_REG(4) BB_SOFTMAX_REG(8) BB_SOFTMAX_REG(16)
+#undef BB_SOFTMAX_REG
+  if (ld <= OPS_ROW_LDS)
+    BB_LAUNCH(k_attn_softmax<true>, grid, dim3(64 * SM_WAVES), (size_t)ld * 4, s, scores, n0, n_heads, ld);
+  else
+    BB_LAUNCH(k_attn_softmax<false>, grid, dim3(64 * SM_WAVES), 0, s, scores, n0, n_heads, ld);
+  return hipGetLastError();
+}
+
 hipError_t launch_attn_pv(hipStream_t s, float* scores, const float* vc, int n0, int T, int n_heads, int n_kv, int hd,
                           float* out) {
-  const int ld = n0 + T;
-  if (T >= AT_PV_MIN_T && hd == AT_HD && n_heads / n_kv <= AT_PV_ITEMS) {
+  const int ld = attn_ld(n0 + T);
+  if (attn_batch(T, hd, n_heads, n_kv)) {
     // a batch: every row's softmax, then P·V in tiles of (tokens x heads of one kv head)
-    if (ld <= OPS_ROW_LDS)
-      BB_LAUNCH(k_attn_softmax<true>, dim3(n_heads, T), dim3(64 * SM_WAVES), (size_t)ld * 4, s, scores, n0, n_heads, ld);
-    else
-      BB_LAUNCH(k_attn_softmax<false>, dim3(n_heads, T), dim3(64 * SM_WAVES), 0, s, scores, n0, n_heads, ld);
-    const hipError_t e = hipGetLastError();
+    const hipError_t e = launch_attn_softmax(s, scores, n0, T, n_heads, ld);
     if (e != hipSuccess) return e;
-    const int TT = at_tokens(n_heads / n_kv, AT_PV_ITEMS);
-    BB_LAUNCH(k_attn_pv_tile, dim3(n_kv, (unsigned)((T + TT - 1) / TT)), dim3(256), 0, s, scores, vc, n0, T, n_heads,
-              n_kv, ld, out);
+    const int TT = at_tokens(n_heads / n_kv, 16);
+    const int tiles = (T + TT - 1) / TT;
+    if (tiles * n_kv * 2 >= 2048)
+      BB_LAUNCH(k_attn_pv_mfma<2>, dim3(n_kv, (unsigned)((tiles + 1) / 2)), dim3(256), 0, s, scores, vc, n0, T, n_heads,
+                n_kv, ld, out);
+    else
+      BB_LAUNCH(k_attn_pv_mfma<4>, dim3(n_kv, (unsigned)tiles), dim3(256), 0, s, scores, vc, n0, T, n_heads, n_kv, ld,
+                out);
     return hipGetLastError();
   }
   const int G = n_heads / n_kv;
   if (hd == AT_HD && ld >= PVL_MIN_LD && (G == 1 || G == 2 || G == 4 || G == 8 || G == 16)) {
     // long rows: the softmax, then P·V with the values streamed through LDS (k_attn_pv_long)
-    if (ld <= OPS_ROW_LDS)
-      BB_LAUNCH(k_attn_softmax<true>, dim3(n_heads, T), dim3(64 * SM_WAVES), (size_t)ld * 4, s, scores, n0, n_heads, ld);
-    else
-      BB_LAUNCH(k_attn_softmax<false>, dim3(n_heads, T), dim3(64 * SM_WAVES), 0, s, scores, n0, n_heads, ld);
-    const hipError_t e = hipGetLastError();
+    const hipError_t e = launch_attn_softmax(s, scores, n0, T, n_heads, ld);
     if (e != hipSuccess) return e;
     const dim3 grid(n_kv, G, T);
     auto blk = [](int np) { return dim3(64 * (1 + np)); };  // the chain wave and the producers
