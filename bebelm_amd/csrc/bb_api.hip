@@ -509,11 +509,40 @@ bool tiled_input(const bb_dense* d, size_t T) {
   return bb::proj_applies(d->gu, T, d->H) && bb::proj_applies(d->dn, T, d->F);
 }
 
+size_t row_bytes_of(const bb_tensor* w) { return w->dims[0] / 256 * (w->dtype == BB_Q4_K ? 144 : 210); }
+
+// One token through a layer's sub-layer whose projections prepare their activations themselves
+// (bb_row1.hip): from the f32 row x, or from the residual stream before the layer boundary.
+bool row1_ok(const bb_dense* d) {
+  return quantised(d->gate) && d->gate->dtype == d->up->dtype && quantised(d->down) && bb::row1_applies(d->H, true) &&
+         bb::row1_applies(d->F, false);
+}
+bb::Row1Job row1_job(const bb_tensor* w, float* y) {
+  return {w->dev, nullptr, row_bytes_of(w), (int)w->dims[1], (int)w->dtype, 0, y};
+}
+// y = W·x of one token from the f32 row x.
+void row1_project(bb_ctx* c, const bb_tensor* w, const float* x, float* y) {
+  launch(c, bb::K_ROWS_Q8, [&] {
+    return bb::launch_row1(c->stream, bb::Row1In{x}, bb::Row1Jobs{1, {row1_job(w, y)}}, (int)w->dims[0]);
+  });
+}
+
 // ---- dense FFN on device pointers (model.rs:459-469 / :262-278) --------------------------------
 // xq_in (may be null): x's Q8, already computed (the decoder's fused residual + rmsnorm) in the
-// layout tiled_input asks for.
-void dense_forward_dev(bb_ctx* c, bb_dense* d, const float* x, size_t T, float* out, const bb::Q8Bufs* xq_in = nullptr) {
+// layout tiled_input asks for. one (may be null; T = 1 and row1_ok): the input instead of x.
+void dense_forward_dev(bb_ctx* c, bb_dense* d, const float* x, size_t T, float* out, const bb::Q8Bufs* xq_in = nullptr,
+                       const bb::Row1In* one = nullptr) {
   const size_t H = d->H, F = d->F;
+  if (T == 1 && !xq_in && row1_ok(d)) {
+    const bb::Row1In in = one ? *one : bb::Row1In{x};
+    float* act = reinterpret_cast<float*>(ensure_ws(c, F * 4));
+    launch(c, bb::K_ROWS_Q8, [&] {
+      return bb::launch_row1_swiglu(c->stream, in, d->gate->dev, d->up->dev, (int)d->gate->dtype, row_bytes_of(d->gate),
+                                    (int)H, (int)F, act);
+    });
+    row1_project(c, d->down, act, out);
+    return;
+  }
   const bool tiled = tiled_input(d, T);
   uint8_t* base = nullptr;
   for (int pass = 0; pass < 2; ++pass) {
@@ -876,10 +905,25 @@ bool tiled_input(const bb_attn_op* op, size_t T) {
 }
 
 // model.rs:399-427 (T == 1) and :190-216 (T > 1) on device pointers; state [(L-1)][H] is updated.
-// xq_in (may be null): x's Q8 in the layout tiled_input asks for.
+// xq_in (may be null): x's Q8 in the layout tiled_input asks for. one (may be null; T = 1 and
+// row1_ok): the input instead of x.
+bool row1_ok(const bb_conv_op* op) {
+  return quantised(op->in_proj) && quantised(op->out_proj) && bb::row1_applies(op->H, true) && op->L >= 2 &&
+         op->L <= bb::R1_L_MAX;
+}
 void conv_forward_dev(bb_ctx* c, bb_conv_op* op, float* state, const float* x, size_t T, float* out,
-                      const bb::Q8Bufs* xq_in = nullptr) {
+                      const bb::Q8Bufs* xq_in = nullptr, const bb::Row1In* one = nullptr) {
   const size_t H = op->H;
+  if (T == 1 && !xq_in && row1_ok(op)) {
+    const bb::Row1In in = one ? *one : bb::Row1In{x};
+    float* y = reinterpret_cast<float*>(ensure_ws(c, H * 4));
+    launch(c, bb::K_CONV, [&] {
+      return bb::launch_row1_conv(c->stream, in, op->in_proj->dev, (int)op->in_proj->dtype, row_bytes_of(op->in_proj),
+                                  (int)H, bb::Row1Conv{op->conv_w, state, op->L}, y);
+    });
+    row1_project(c, op->out_proj, y, out);
+    return;
+  }
   uint8_t* base = nullptr;
   for (int pass = 0; pass < 2; ++pass) {
     Carve cv{base};
@@ -929,9 +973,15 @@ void ensure_rope(bb_ctx* c, bb_attn_op* op, size_t rows) {
 }
 
 // model.rs:430-456 (T == 1) and :222-259 (T > 1) on device pointers: the T new keys / values
-// are projected straight into the cache rows n .. n+T-1.
+// are projected straight into the cache rows n .. n+T-1. one (may be null; T = 1 and row1_ok): the
+// input instead of x.
+bool row1_ok(const bb_attn_op* op) {
+  return quantised(op->q) && quantised(op->k) && quantised(op->v) && quantised(op->o) &&
+         bb::row1_applies(op->H, true) && bb::row1_applies((size_t)op->NH * op->HD, false);
+}
 void attn_forward_dev(bb_ctx* c, bb_attn_op* op, bb_kv_cache* kv, size_t pos0, const float* x, size_t T, float* out,
-                      const bb::Q8Bufs* xq_in = nullptr) {
+                      const bb::Q8Bufs* xq_in = nullptr, const bb::Row1In* one = nullptr) {
+  const bool row1 = T == 1 && !xq_in && row1_ok(op);
   const size_t H = op->H, NH = op->NH, NKV = op->NKV, HD = op->HD, KV = NKV * HD, QD = NH * HD;
   const size_t n0 = kv->n;
   ensure_rope(c, op, pos0 + T);
@@ -956,13 +1006,20 @@ void attn_forward_dev(bb_ctx* c, bb_attn_op* op, bb_kv_cache* kv, size_t pos0, c
                       (((op->q_p.w || op->k_p.w || op->v_p.w) && !tin) || (op->o_p.w && !tout));
     if (gemm) rb = one_group(c, grp, T);
     const bb::RouteBufs* rbp = gemm ? &rb : nullptr;
-    // x's Q8 once for the three projections, or as given
-    const bb::Q8Bufs xqv = xq_in ? *xq_in : xq;
-    if (!xq_in && (quantised(op->q) || quantised(op->k) || quantised(op->v)))
-      launch(c, bb::K_QUANT, [&] { return bb::launch_quantize(c->stream, x, T, H, xq); });
-    project_dev(c, op->q, op->q_p, rbp, H, QD, x, T, q, xqv, true);
-    project_dev(c, op->k, op->k_p, rbp, H, KV, x, T, kn, xqv, true);
-    project_dev(c, op->v, op->v_p, rbp, H, KV, x, T, vn, xqv, true);
+    if (row1) {
+      launch(c, bb::K_ROWS_Q8, [&] {
+        return bb::launch_row1(c->stream, one ? *one : bb::Row1In{x},
+                               bb::Row1Jobs{3, {row1_job(op->q, q), row1_job(op->k, kn), row1_job(op->v, vn)}}, (int)H);
+      });
+    } else {
+      // x's Q8 once for the three projections, or as given
+      const bb::Q8Bufs xqv = xq_in ? *xq_in : xq;
+      if (!xq_in && (quantised(op->q) || quantised(op->k) || quantised(op->v)))
+        launch(c, bb::K_QUANT, [&] { return bb::launch_quantize(c->stream, x, T, H, xq); });
+      project_dev(c, op->q, op->q_p, rbp, H, QD, x, T, q, xqv, true);
+      project_dev(c, op->k, op->k_p, rbp, H, KV, x, T, kn, xqv, true);
+      project_dev(c, op->v, op->v_p, rbp, H, KV, x, T, vn, xqv, true);
+    }
     const float2* rope = op->rope + pos0 * (HD / 2);
     launch(c, bb::K_NORM_ROPE, [&] {
       return bb::launch_norm_rope(c->stream, q, (int)T, (int)NH, (int)HD, op->q_norm, op->eps, rope, kn, (int)NKV,
@@ -974,7 +1031,8 @@ void attn_forward_dev(bb_ctx* c, bb_attn_op* op, bb_kv_cache* kv, size_t pos0, c
     launch(c, bb::K_ATTN_PV, [&] {
       return bb::launch_attn_pv(c->stream, scores, kv->v, (int)n0, (int)T, (int)NH, (int)NKV, (int)HD, attn);
     });
-    project_dev(c, op->o, op->o_p, rbp, QD, H, attn, T, out, aq);
+    if (row1) row1_project(c, op->o, attn, out);
+    else project_dev(c, op->o, op->o_p, rbp, QD, H, attn, T, out, aq);
   }
   kv->n = n0 + T;
 }
@@ -1549,11 +1607,20 @@ int bb_stack_forward(bb_ctx* c, bb_stack* s, const float* x, size_t T, float* h_
       s->cap_T = T;
     }
     with_io(c, loc, {{x, T * H * 4, true, false}, {h_out, T * H * 4, false, true}}, [&](std::vector<void*>& d) {
-      float* h = s->h;       // the residual stream; at a boundary that routes, h_out is the other buffer
-      float* h_alt = s->h2;
-      check_hip(hipMemcpyAsync(h, d[0], T * H * 4, hipMemcpyDeviceToDevice, c->stream), "h copy");
+      // the residual stream: the input, then s->h and s->h2 in turn (every boundary writes the one it
+      // does not read), the last boundary the output
+      const float* h = static_cast<const float*>(d[0]);
+      float* const out = static_cast<float*>(d[1]);
       const size_t nl = s->layers.size();
-      if (nl)
+      if (nl == 0) {
+        check_hip(hipMemcpyAsync(out, h, T * H * 4, hipMemcpyDeviceToDevice, c->stream), "h copy");
+        return;
+      }
+      auto next_h = [&] { return h == s->h ? s->h2 : s->h; };
+      // one token: a dense layer takes the boundary before it as its input (row1_ok)
+      auto dense1 = [&](size_t l) { return T == 1 && s->layers[l].dense && row1_ok(s->layers[l].dense); };
+      bb::Row1In one{h, nullptr, s->layers[0].ffn_norm, s->eps, nullptr};
+      if (!dense1(0))
         launch(c, bb::K_RMSNORM,
                [&] { return bb::launch_rmsnorm(c->stream, h, s->layers[0].ffn_norm, s->eps, H, T, s->normed); });
       const PreRoute pre{s->logits, bb::XQBufs{s->xq_q, s->xq_sx, s->xq_pairs}};
@@ -1562,12 +1629,13 @@ int bb_stack_forward(bb_ctx* c, bb_stack* s, const float* x, size_t T, float* h_
         const bb_layer_desc& L = s->layers[l];
         // the layer's FFN on normed, then h += its output and the next layer's rmsnorm, fused;
         // before an MoE layer of a few tokens on the GEMV path the same kernel also takes its
-        // router logits
+        // router logits, and before a dense layer of one token the next layer does it all
         const float* next_gain = l + 1 < nl ? s->layers[l + 1].ffn_norm : nullptr;
         const bb_moe* nm = l + 1 < nl ? s->layers[l + 1].moe : nullptr;
         const bool route_next = nm && T <= (size_t)bb::ROUTE_IN_GATEUP_MAX_T &&
                                 T * (size_t)nm->K < c->batched_min_entries && H % 128 == 0 && nm->E <= 32 &&
                                 nm->K <= 8;
+        const bool dense_next = l + 1 < nl && dense1(l + 1);
         const float* slots = nullptr;
         const float* wts = nullptr;
         int K = 0;
@@ -1577,23 +1645,31 @@ int bb_stack_forward(bb_ctx* c, bb_stack* s, const float* x, size_t T, float* h_
           wts = w.rb.wts;
           K = L.moe->K;
         } else {
-          dense_forward_dev(c, L.dense, s->normed, T, s->ffn);
+          dense_forward_dev(c, L.dense, s->normed, T, s->ffn, nullptr, dense1(l) ? &one : nullptr);
+          if (dense1(l) && one.add) h = one.h_out;
         }
         const float* ffn = L.moe ? nullptr : s->ffn;
+        routed = route_next;
+        if (dense_next && ffn) {
+          one = bb::Row1In{h, ffn, next_gain, s->eps, next_h()};
+          continue;
+        }
+        float* const ho = l + 1 < nl ? next_h() : out;
         if (route_next) {
           launch(c, bb::K_RESIDUAL_ROUTE, [&] {
-            return bb::launch_residual_norm_route(c->stream, h, h_alt, slots, wts, K, ffn, next_gain, s->eps, (int)H,
+            return bb::launch_residual_norm_route(c->stream, h, ho, slots, wts, K, ffn, next_gain, s->eps, (int)H,
                                                   (int)T, s->normed, nm->router_cm, nm->E, s->logits, pre.xq);
           });
-          std::swap(h, h_alt);
         } else {
+          // (before a dense layer after an MoE layer: the combine here, the rmsnorm there)
           launch(c, bb::K_RESIDUAL_NORM, [&] {
-            return bb::launch_residual_norm(c->stream, h, slots, wts, K, ffn, next_gain, s->eps, H, T, s->normed);
+            return bb::launch_residual_norm(c->stream, h, ho, slots, wts, K, ffn, dense_next ? nullptr : next_gain,
+                                            s->eps, H, T, s->normed);
           });
         }
-        routed = route_next;
+        h = ho;
+        if (dense_next) one = bb::Row1In{h, nullptr, next_gain, s->eps, nullptr};
       }
-      check_hip(hipMemcpyAsync(d[1], h, T * H * 4, hipMemcpyDeviceToDevice, c->stream), "h copy");
     });
   });
 }
@@ -2028,8 +2104,9 @@ const uint32_t* model_tokens(bb_ctx* c, bb_model* m, const uint32_t* host, size_
 
 // Model::run_layers (T == 1, model.rs:105-130) / run_layers_batch (T > 1, :146-181): embeds
 // the tokens (device ids) at positions k->pos.., runs every layer (updating the cache's conv
-// states and KV histories) and leaves the final hidden states in m->h.
-void model_run_dev(bb_ctx* c, bb_model* m, bb_cache* k, const uint32_t* tokens, size_t T) {
+// states and KV histories) and leaves the final hidden states in m->h. final_q8 (may be null; T = 1):
+// set when the last boundary also took the final rmsnorm and left its Q8 in m->nq.
+void model_run_dev(bb_ctx* c, bb_model* m, bb_cache* k, const uint32_t* tokens, size_t T, bool* final_q8 = nullptr) {
   for (bb_kv_cache* kv : k->kv)
     if (kv) kv_reserve(c, kv, kv->n + T);
   model_buffers(c, m, T);
@@ -2041,42 +2118,54 @@ void model_run_dev(bb_ctx* c, bb_model* m, bb_cache* k, const uint32_t* tokens, 
   // Each layer boundary (h += sub-layer output, then the next rmsnorm) is one launch of
   // k_residual_norm, which also writes the normed rows' Q8 when the next sub-layer projects
   // them (conv, attention, dense FFN; the MoE route quantises its input itself) in the layout that
-  // it reads, or, before an
-  // MoE layer of a few tokens, of k_residual_norm_route, which also takes the layer's router
-  // logits and XQ records.
+  // it reads, or, before an MoE layer of a few tokens, of k_residual_norm_route, which also takes
+  // the layer's router logits and XQ records. For one token a sub-layer whose projections prepare
+  // their input themselves (row1_ok) takes the boundary as its input, with no launch of its own.
   const bool fused = H <= (size_t)bb::GU_H_MAX && m->nq.q;
-  auto op_tiled = [&](size_t i) {
-    return m->layers[i].conv ? tiled_input(m->layers[i].conv, T) : tiled_input(m->layers[i].attn, T);
+  const size_t n_layers = m->layers.size();
+  auto op_row1 = [&](size_t i) {
+    const auto& L = m->layers[i];
+    return T == 1 && fused && (L.conv ? row1_ok(L.conv) : row1_ok(L.attn));
   };
-  auto boundary = [&](const float* gain, bool q8, bool tiled) {
+  auto op_tiled = [&](size_t i) {
+    const auto& L = m->layers[i];
+    return L.conv ? tiled_input(L.conv, T) : tiled_input(L.attn, T);
+  };
+  // a boundary of its own: h += add (m->tmp or null), then the rmsnorm with gain unless it is null
+  auto boundary = [&](const float* add, const float* gain, bool q8, bool tiled) {
     m->nq.tiled = tiled;
-    if (fused) {
+    if (fused && add) {
       launch(c, bb::K_RESIDUAL_NORM, [&] {
-        return bb::launch_residual_norm(c->stream, m->h, nullptr, nullptr, 0, m->tmp, gain, m->eps, H, T, m->normed,
+        return bb::launch_residual_norm(c->stream, m->h, m->h, nullptr, nullptr, 0, add, gain, m->eps, H, T, m->normed,
                                         q8 && gain ? m->nq : bb::Q8Bufs{});
       });
       return;
     }
-    launch(c, bb::K_ELEMWISE, [&] {
-      return bb::launch_elementwise(c->stream, bb::EW_ADD_ASSIGN, m->h, m->tmp, nullptr, 0.0f, T * H);
-    });
+    if (fused) {
+      launch(c, bb::K_RMSNORM,
+             [&] { return bb::launch_rmsnorm_q8(c->stream, m->h, gain, m->eps, H, T, m->normed, m->nq); });
+      return;
+    }
+    if (add)
+      launch(c, bb::K_ELEMWISE, [&] {
+        return bb::launch_elementwise(c->stream, bb::EW_ADD_ASSIGN, m->h, add, nullptr, 0.0f, T * H);
+      });
     if (gain) launch(c, bb::K_RMSNORM, [&] { return bb::launch_rmsnorm(c->stream, m->h, gain, m->eps, H, T, m->normed); });
   };
   const bb::Q8Bufs* nq = fused ? &m->nq : nullptr;
-  const size_t n_layers = m->layers.size();
-  m->nq.tiled = op_tiled(0);
-  if (fused)
-    launch(c, bb::K_RMSNORM, [&] {
-      return bb::launch_rmsnorm_q8(c->stream, m->h, m->layers[0].attn_norm, m->eps, H, T, m->normed, m->nq);
-    });
-  else
-    launch(c, bb::K_RMSNORM, [&] {
-      return bb::launch_rmsnorm(c->stream, m->h, m->layers[0].attn_norm, m->eps, H, T, m->normed);
-    });
+  const float* add = nullptr;  // the sub-layer output not yet added to h
   for (size_t i = 0; i < n_layers; ++i) {
     auto& L = m->layers[i];
-    if (L.conv) conv_forward_dev(c, L.conv, k->conv[i], m->normed, T, m->tmp, nq);
-    else attn_forward_dev(c, L.attn, k->kv[i], k->pos, m->normed, T, m->tmp, nq);
+    if (op_row1(i)) {
+      const bb::Row1In in{m->h, add, L.attn_norm, m->eps, m->h2};
+      if (L.conv) conv_forward_dev(c, L.conv, k->conv[i], nullptr, T, m->tmp, nullptr, &in);
+      else attn_forward_dev(c, L.attn, k->kv[i], k->pos, nullptr, T, m->tmp, nullptr, &in);
+      if (add) std::swap(m->h, m->h2);
+    } else {
+      boundary(add, L.attn_norm, true, op_tiled(i));
+      if (L.conv) conv_forward_dev(c, L.conv, k->conv[i], m->normed, T, m->tmp, nq);
+      else attn_forward_dev(c, L.attn, k->kv[i], k->pos, m->normed, T, m->tmp, nq);
+    }
     // before an MoE layer of a few tokens on the GEMV path the boundary also takes the layer's
     // router logits and its input's XQ records, and the gate/up GEMV only gates
     const bb_moe* mo = L.moe;
@@ -2091,14 +2180,20 @@ void model_run_dev(bb_ctx* c, bb_model* m, bb_cache* k, const uint32_t* tokens, 
       std::swap(m->h, m->h2);
       const PreRoute pre{m->logits, m->xq};
       moe_forward_dev(c, L.moe, m->normed, T, m->tmp, nullptr, true, &pre);
+    } else if (T == 1 && fused && L.dense && row1_ok(L.dense)) {
+      const bb::Row1In in{m->h, m->tmp, L.ffn_norm, m->eps, m->h2};
+      dense_forward_dev(c, L.dense, nullptr, T, m->tmp, nullptr, &in);
+      std::swap(m->h, m->h2);
     } else {
-      boundary(L.ffn_norm, L.dense != nullptr, L.dense && tiled_input(L.dense, T));
+      boundary(m->tmp, L.ffn_norm, L.dense != nullptr, L.dense && tiled_input(L.dense, T));
       if (L.moe) moe_forward_dev(c, L.moe, m->normed, T, m->tmp, nullptr);
       else dense_forward_dev(c, L.dense, m->normed, T, m->tmp, nq);
     }
-    const bool more = i + 1 < n_layers;
-    boundary(more ? m->layers[i + 1].attn_norm : nullptr, true, more && op_tiled(i + 1));
+    add = m->tmp;
   }
+  const bool final_here = final_q8 && fused && T == 1 && add;
+  if (add) boundary(add, final_here ? m->final_norm : nullptr, final_here, false);
+  if (final_q8) *final_q8 = final_here;
   k->pos += T;
 }
 
@@ -2369,8 +2464,16 @@ int bb_model_forward_step(bb_ctx* c, bb_model* m, uint32_t token, bb_cache* k, f
     need_loc(loc);
     set_device(c);
     with_io(c, loc, {{logits, m->vocab * 4, false, true}}, [&](std::vector<void*>& d) {
-      model_run_dev(c, m, k, model_tokens(c, m, &token, 1), 1);
-      logits_dev(c, m->tok_embd, m->final_norm, m->eps, m->h, static_cast<float*>(d[0]));
+      bool normed = !quantised(m->tok_embd);  // (a quantised head reads the last boundary's Q8)
+      bool* want = normed ? nullptr : &normed;
+      model_run_dev(c, m, k, model_tokens(c, m, &token, 1), 1, want);
+      if (want && normed)
+        launch(c, bb::K_ROWS_Q8, [&] {
+          return bb::launch_rows_q8(c->stream, (int)m->tok_embd->dtype, m->tok_embd->dev, m->row_bytes, m->H / 256,
+                                    m->vocab, m->nq, m->H, 1, static_cast<float*>(d[0]), m->vocab, 1);
+        });
+      else
+        logits_dev(c, m->tok_embd, m->final_norm, m->eps, m->h, static_cast<float*>(d[0]));
     });
   });
 }

@@ -267,6 +267,46 @@ hipError_t launch_rows_f32(hipStream_t s, int dtype, const uint8_t* w, size_t n_
 hipError_t launch_fused_rows_f32(hipStream_t s, int dtype, const uint8_t* w, size_t row_bytes, int nb, size_t n_rows,
                                  const float* x, float* y);
 
+// ---- one token's projections with their neighbours (bb_row1.hip) ----
+// The token's activations: Q8 of the row x, or (gain set) of rmsnorm(h, gain, eps) with h = x + add
+// (add may be null; else h goes to h_out, which must not alias x).
+struct Row1In {
+  const float* x;
+  const float* add = nullptr;
+  const float* gain = nullptr;
+  float eps = 0.0f;
+  float* h_out = nullptr;
+};
+// A Q4_K / Q6_K matrix in GGUF rows: n_rows outputs to y (w2: the up matrix of a SwiGLU pair).
+// first: its first block in the launch, set by the launcher.
+struct Row1Job {
+  const uint8_t *w, *w2;
+  size_t row_bytes;
+  int n_rows, dt, first;
+  float* y;
+};
+struct Row1Jobs {
+  int n;
+  Row1Job job[3];
+};
+// The short conv: taps [channel][L] and the cache state [L-1][channels], updated.
+struct Row1Conv {
+  const float* w;
+  float* state;
+  int L;
+};
+constexpr int R1_L_MAX = 4;        // longest filter
+constexpr int ROW1_N_MAX = 8192;   // longest row (GU_H_MAX with the rmsnorm)
+bool row1_applies(size_t n, bool norm);
+// y = W·x for up to three matrices of rows of n (sums from -0.0, matvec's).
+hipError_t launch_row1(hipStream_t s, const Row1In& in, Row1Jobs jobs, int n);
+// The conv operator's in_proj [H -> 3H] and conv: y[H] = C·conv (model.rs:399-421), state updated.
+hipError_t launch_row1_conv(hipStream_t s, const Row1In& in, const uint8_t* w, int dt, size_t row_bytes, int H,
+                            const Row1Conv& cv, float* y);
+// y[n_out] = silu(gate·x)·(up·x).
+hipError_t launch_row1_swiglu(hipStream_t s, const Row1In& in, const uint8_t* gate, const uint8_t* up, int dt,
+                              size_t row_bytes, int n, int n_out, float* y);
+
 enum ElemOp : int { EW_SWIGLU = 0, EW_SIGMOID, EW_ADD_SCALED, EW_ADD_ASSIGN };
 hipError_t launch_elementwise(hipStream_t s, int op, float* out, const float* a, const float* b, float scalar,
                               size_t n);
@@ -276,9 +316,11 @@ hipError_t launch_rmsnorm(hipStream_t s, const float* x, const float* gain, floa
 // The same, and the Q8 of each normed row into q (n <= GU_H_MAX, n % 256 == 0; out may be null).
 hipError_t launch_rmsnorm_q8(hipStream_t s, const float* x, const float* gain, float eps, size_t n, size_t n_vec,
                              float* out, Q8Bufs q);
-// h += (slots, wts, K) combine or ffn row; then normed = rmsnorm(h, gain) unless gain is null.
-hipError_t launch_residual_norm(hipStream_t s, float* h, const float* slots, const float* wts, int K, const float* ffn,
-                                const float* gain, float eps, size_t n, size_t n_vec, float* normed, Q8Bufs q = Q8Bufs{});
+// h_out = h_in + the (slots, wts, K) combine or ffn row (h_out may be h_in); then normed =
+// rmsnorm(h_out, gain) unless gain is null.
+hipError_t launch_residual_norm(hipStream_t s, const float* h_in, float* h_out, const float* slots, const float* wts,
+                                int K, const float* ffn, const float* gain, float eps, size_t n, size_t n_vec,
+                                float* normed, Q8Bufs q = Q8Bufs{});
 
 // ---- decoder-layer operators (bb_ops.hip) ----
 constexpr int OPS_HD_MAX = 256;     // head_dim bound of the attention kernels

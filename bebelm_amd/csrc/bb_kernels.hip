@@ -452,12 +452,13 @@ __global__ void __launch_bounds__(256) k_rmsnorm(const float* __restrict__ x, co
 // selection order from +0.0 (model.rs:550-553 / :362-369) or a dense FFN output row; then the
 // next layer's rmsnorm of h (as k_rmsnorm: the same f64 partial sums and tree) unless gain is
 // null. One launch instead of combine, add_assign and rmsnorm.
-__global__ void __launch_bounds__(256) k_residual_norm(float* __restrict__ h, const float* __restrict__ slots,
+__global__ void __launch_bounds__(256) k_residual_norm(const float* h_in, float* h_out, const float* __restrict__ slots,
                                                        const float* __restrict__ wts, int K,
                                                        const float* __restrict__ ffn, const float* __restrict__ gain,
                                                        float eps, size_t n, float* __restrict__ normed, Q8Bufs q) {
   const size_t t = blockIdx.x;
-  float* hv = h + t * n;
+  const float* hi = h_in + t * n;  // (h_out may be h_in: a thread reads its elements before it writes them)
+  float* hv = h_out + t * n;
   // thread j takes elements j, j+256, ... (k_rmsnorm's order); every load is issued before the
   // first use, so the block waits for memory once
   constexpr int NI = GU_H_MAX / 256;
@@ -481,7 +482,7 @@ __global__ void __launch_bounds__(256) k_residual_norm(float* __restrict__ h, co
 #pragma unroll
     for (int it = 0; it < NI; ++it) {
       const size_t i = min((size_t)(threadIdx.x + 256 * it), n - 1);
-      hr[it] = hv[i];
+      hr[it] = hi[i];
       yr[it] = 0.0f;
     }
 #pragma unroll
@@ -494,7 +495,7 @@ __global__ void __launch_bounds__(256) k_residual_norm(float* __restrict__ h, co
 #pragma unroll
     for (int it = 0; it < NI; ++it) {
       const size_t i = min((size_t)(threadIdx.x + 256 * it), n - 1);
-      hr[it] = hv[i];
+      hr[it] = hi[i];
       yr[it] = ffn[t * n + i];
     }
   }
@@ -551,12 +552,13 @@ __global__ void __launch_bounds__(256) k_residual_norm(float* __restrict__ h, co
   }
 }
 
-hipError_t launch_residual_norm(hipStream_t s, float* h, const float* slots, const float* wts, int K, const float* ffn,
+hipError_t launch_residual_norm(hipStream_t s, const float* h_in, float* h_out, const float* slots, const float* wts, int K, const float* ffn,
                                 const float* gain, float eps, size_t n, size_t n_vec, float* normed, Q8Bufs q) {
   if (n_vec == 0) return hipSuccess;
   if (n > (size_t)GU_H_MAX || K > 8) return hipErrorInvalidValue;  // the kernel's register tiles
   if (q.q && (!gain || n % QK != 0)) return hipErrorInvalidValue;
-  BB_LAUNCH(k_residual_norm, dim3((unsigned)n_vec), dim3(256), 0, s, h, slots, wts, K, ffn, gain, eps, n, normed, q);
+  BB_LAUNCH(k_residual_norm, dim3((unsigned)n_vec), dim3(256), 0, s, h_in, h_out, slots, wts, K, ffn, gain, eps, n,
+            normed, q);
   return hipGetLastError();
 }
 
