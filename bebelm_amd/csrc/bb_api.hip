@@ -118,6 +118,7 @@ struct bb_ctx {
   double kernel_ms[bb::K_COUNT] = {};
   int64_t launches[bb::K_COUNT] = {};
   size_t batched_min_entries = 64;  // T*k from which MoE calls take the grouped-GEMM path
+  bool batched_default = true;      // (not set by the caller)
   int n_cu = 256;                   // compute units of the device
 };
 
@@ -341,6 +342,17 @@ bool moe_act_pad(const bb_moe* m, size_t T) {
          bb::down16_applies((int)m->dn_dtype, (int)T, (int)m->H, (int)m->F, (int)m->E, (int)m->K);
 }
 
+// Whether a call of T tokens takes the grouped-GEMM kernels. Unless the caller set the line, layers
+// whose batch both decode-batch kernels serve take them from 32 entries: config 2's layer, GEMV path
+// and here, 7 tokens 45 and 42 us, 8 tokens 46.8 and 42.9 (Q6_K down 52.8 and 52.4), 12 tokens 57.6
+// and 46.2 (65.5 and 54.7), 15 tokens 67.3 and 49.5; at 6 tokens Q6_K 47.9 and 51.1.
+constexpr size_t DECODE_BATCH_MIN_ENTRIES = 32;
+bool moe_batched(const bb_ctx* c, const bb_moe* m, size_t T) {
+  const size_t n_ent = T * (size_t)m->K;
+  return n_ent >= c->batched_min_entries ||
+         (c->batched_default && n_ent >= DECODE_BATCH_MIN_ENTRIES && moe_act_pad(m, T));
+}
+
 MoeWs carve_moe(bb_ctx* c, const bb_moe* m, size_t T, bool batched, const WsRegion* fixed = nullptr) {
   const size_t H = m->H, F = m->F, E = m->E, K = m->K;
   for (int pass = 0; pass < 2; ++pass) {
@@ -394,7 +406,7 @@ MoeWs moe_forward_dev(bb_ctx* c, bb_moe* m, const float* x, size_t T, float* out
                       bool combine = true, const PreRoute* pre = nullptr, const WsRegion* fixed = nullptr) {
   need(T >= 1, BB_ERR_ARG, "T must be >= 1");
   const size_t n_ent = T * (size_t)m->K;
-  const bool batched = n_ent >= c->batched_min_entries;
+  const bool batched = moe_batched(c, m, T);
   if (batched)
     need(n_ent <= (size_t)bb::PF_MAX_ENTRIES, BB_ERR_RANGE, "this path routes at most 32768 (token, slot) entries per call");
   else
@@ -434,10 +446,12 @@ MoeWs moe_forward_dev(bb_ctx* c, bb_moe* m, const float* x, size_t T, float* out
   } else {
     const int batch_mode = T > 1;
     const int max_hit = (int)std::min<size_t>((size_t)m->E, n_ent);
-    // a few tokens: every gate/up block routes them itself (or only gates them, from logits
-    // computed before the call)
-    const bool route_in = T <= (size_t)bb::ROUTE_IN_GATEUP_MAX_T;
-    need(!pre || route_in, BB_ERR_ARG, "routes computed before the call serve at most 4 tokens");
+    // one or two tokens: every gate/up block routes them itself (or, up to four, only gates them, from
+    // logits computed before the call). With three the blocks' own routes already cost more than a
+    // launch (config 2's layer: 3 tokens 38 us against 34, 4 tokens 44 against 37).
+    need(!pre || T <= (size_t)bb::ROUTE_IN_GATEUP_MAX_T, BB_ERR_ARG,
+         "routes computed before the call serve at most 4 tokens");
+    const bool route_in = pre || T <= 2;
     if (!route_in)
       launch(c, bb::K_ROUTE, [&] {
         return bb::launch_route(c->stream, m->router_cm, m->bias_dev, x, (int)T, m->H, m->E, m->K, 1, w.xq, w.rb);
@@ -1156,6 +1170,7 @@ int bb_ctx_set_batched_min_entries(bb_ctx* c, size_t min_entries) {
   return guard([&] {
     need_ctx(c);
     c->batched_min_entries = min_entries;
+    c->batched_default = false;
   });
 }
 
@@ -1633,8 +1648,7 @@ int bb_stack_forward(bb_ctx* c, bb_stack* s, const float* x, size_t T, float* h_
         const float* next_gain = l + 1 < nl ? s->layers[l + 1].ffn_norm : nullptr;
         const bb_moe* nm = l + 1 < nl ? s->layers[l + 1].moe : nullptr;
         const bool route_next = nm && T <= (size_t)bb::ROUTE_IN_GATEUP_MAX_T &&
-                                T * (size_t)nm->K < c->batched_min_entries && H % 128 == 0 && nm->E <= 32 &&
-                                nm->K <= 8;
+                                !moe_batched(c, nm, T) && H % 128 == 0 && nm->E <= 32 && nm->K <= 8;
         const bool dense_next = l + 1 < nl && dense1(l + 1);
         const float* slots = nullptr;
         const float* wts = nullptr;
@@ -2170,8 +2184,7 @@ void model_run_dev(bb_ctx* c, bb_model* m, bb_cache* k, const uint32_t* tokens, 
     // router logits and its input's XQ records, and the gate/up GEMV only gates
     const bb_moe* mo = L.moe;
     const bool route_here = fused && mo && m->h2 && T <= (size_t)bb::ROUTE_IN_GATEUP_MAX_T &&
-                            T * (size_t)mo->K < c->batched_min_entries && H % 128 == 0 && mo->E <= 32 &&
-                            mo->K <= 8;
+                            !moe_batched(c, mo, T) && H % 128 == 0 && mo->E <= 32 && mo->K <= 8;
     if (route_here) {
       launch(c, bb::K_RESIDUAL_ROUTE, [&] {
         return bb::launch_residual_norm_route(c->stream, m->h, m->h2, nullptr, nullptr, 0, m->tmp, L.ffn_norm, m->eps,

@@ -117,14 +117,12 @@ __device__ __forceinline__ void q4_step_ops(const uint4 qv, int h, const Q4Lane&
 // halves at msb + 32m, lane group g's four at + 8g) by one f16 MFMA per member tile, against
 // weights [64·m_{2g}, 64·m_{2g+1}, m_{2g}, m_{2g+1}]: sm arrives as an exact f32, instead of a
 // third int8 pass over the block (four MFMAs) and a conversion.
-template <int MT, bool MF = false>
-__device__ __forceinline__ void q4_block(const uint8_t* wt, const uint8_t* xb, const float* sb, const uint8_t* msb,
-                                         int row, float (&acc)[MT][4]) {
+// built() runs once the operands no longer need the weight words.
+template <int MT, bool MF = false, class Built>
+__device__ __forceinline__ void q4_tiles(const uint4 hd, const uint4 (&qv)[2], const uint8_t* xb, const float* sb,
+                                         const uint8_t* msb, float (&acc)[MT][4], Built&& built) {
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  const Q4Lane L = q4_lane(*reinterpret_cast<const uint4*>(wt + 16 * row), g);
-  uint4 qv[2];
-#pragma unroll
-  for (int k = 0; k < 2; ++k) qv[k] = *reinterpret_cast<const uint4*>(wt + 1024 * (1 + 2 * g + k) + 16 * row);
+  const Q4Lane L = q4_lane(hd, g);
   v4i Bm[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) Bm[h] = (v4i){L.ms[h], L.ms[h], L.ms[h], L.ms[h]};
@@ -141,6 +139,7 @@ __device__ __forceinline__ void q4_block(const uint8_t* wt, const uint8_t* xb, c
       Dl = __builtin_amdgcn_mfma_i32_16x16x64_i8(ax, Bl, Dl, 0, 0, 0);
       Dm = __builtin_amdgcn_mfma_i32_16x16x64_i8(ax, Bm[s >> 1], Dm, 0, 0, 0);
     }
+    built();
     const float4 sx4 = *reinterpret_cast<const float4*>(sb + 4 * g);
     const float sxv[4] = {sx4.x, sx4.y, sx4.z, sx4.w};
 #pragma unroll
@@ -157,6 +156,7 @@ __device__ __forceinline__ void q4_block(const uint8_t* wt, const uint8_t* xb, c
   v4i Bh[4], Bl[4];
 #pragma unroll
   for (int s = 0; s < 4; ++s) q4_step_ops(qv[s & 1], s >> 1, L, Bh[s], Bl[s]);
+  built();
   v4h bmin;
   if constexpr (MF)
     bmin = (v4h){(_Float16)(64 * L.m[0]), (_Float16)(64 * L.m[1]), (_Float16)L.m[0], (_Float16)L.m[1]};
@@ -190,6 +190,17 @@ __device__ __forceinline__ void q4_block(const uint8_t* wt, const uint8_t* xb, c
   }
 }
 
+// The same with the weight words in LDS (the packed tile-block wt, the lane's row).
+template <int MT, bool MF = false>
+__device__ __forceinline__ void q4_block(const uint8_t* wt, const uint8_t* xb, const float* sb, const uint8_t* msb,
+                                         int row, float (&acc)[MT][4]) {
+  const int g = (threadIdx.x & 63) >> 4;
+  uint4 qv[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) qv[k] = *reinterpret_cast<const uint4*>(wt + 1024 * (1 + 2 * g + k) + 16 * row);
+  q4_tiles<MT, MF>(*reinterpret_cast<const uint4*>(wt + 16 * row), qv, xb, sb, msb, acc, [] {});
+}
+
 // (hi, lo) int8 parts of sc*(q - 32) for four quant bytes q (<= 63): the products are formed
 // in 16-bit lanes (even and odd bytes) and the bytes put back in order.
 __device__ __forceinline__ void q6_split(uint32_t q, uint32_t scp, uint32_t bias, uint32_t& h, uint32_t& l) {
@@ -207,39 +218,40 @@ __device__ __forceinline__ void q6_split(uint32_t q, uint32_t scp, uint32_t bias
   h = __builtin_amdgcn_perm(ho, he, 0x06020400u);
 }
 
+// The weight operands of step c (elements 64c + 16g.. of lane group g) from the lane's ql and qh words
+// of half c / 2 and the dword of the sub-block's scale: elements 64c + 16g + t = 128n + 32gq + 16(g&1)
+// + t with n = c/2, gq = 2(c&1) + g/2 (dequant.rs:122-138): ql[64n + 32(g/2) + 16(g&1) + t] (high
+// nibble when c is odd) and bits 2gq of qh[32n + 16(g&1) + t]; sub-block j = 4c + g.
+__device__ __forceinline__ void q6_step_ops(const uint4 qlv, const uint4 qhv, uint32_t scd, int c, int g, v4i& Bh,
+                                            v4i& Bl) {
+  const uint32_t lsh = 4 * (c & 1), hsh = 2 * (2 * (c & 1) + (g >> 1));
+  const int scj = (int)(int8_t)((scd >> (8 * g)) & 0xffu);
+  const uint32_t scp = ((uint32_t)scj & 0xffffu) * 0x00010001u;
+  const uint32_t bias = ((uint32_t)(-32 * scj) & 0xffffu) * 0x00010001u;
+  const uint32_t qlw[4] = {qlv.x, qlv.y, qlv.z, qlv.w}, qhw[4] = {qhv.x, qhv.y, qhv.z, qhv.w};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t q = ((qlw[k] >> lsh) & 0x0F0F0F0Fu) | (((qhw[k] >> hsh) & 0x03030303u) << 4);
+    uint32_t hh, ll;
+    q6_split(q, scp, bias, hh, ll);
+    Bh[k] = (int)hh;
+    Bl[k] = (int)ll;
+  }
+}
+
 // Q6_K: s = Σ_j sc_j·Σ (q − 32)·x. With a = sc_j·(q − 32) (|a| <= 4096) split as a = 64·h + l,
 // h in [−64, 64] and l in [0, 63] both fit int8: two passes give s = 64·Dh + Dl. Epilogue
 // matmul.rs:641: sx·(d·(float)s).
-template <int MT>
-__device__ __forceinline__ void q6_block(const uint8_t* wt, const uint8_t* xb, const float* sb, int row,
-                                         float (&acc)[MT][4]) {
+// built() runs once the operands no longer need the weight words.
+template <int MT, class Built>
+__device__ __forceinline__ void q6_tiles(const uint4 (&ql)[2], const uint4 (&qh)[2], const uint4 sc, float d,
+                                         const uint8_t* xb, const float* sb, float (&acc)[MT][4], Built&& built) {
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  const uint4 sc = *reinterpret_cast<const uint4*>(wt + 1024 * 12 + 16 * row);
-  const float d = f16_bits_to_f32(*reinterpret_cast<const uint16_t*>(wt + 1024 * 13 + 2 * row));
   v4i Bh[4], Bl[4];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    // elements 64c + 16g + t = 128n + 32gq + 16(g&1) + t with n = c/2, gq = 2(c&1) + g/2
-    // (dequant.rs:122-138): ql[64n + 32(g/2) + 16(g&1) + t] (high nibble when c is odd) and
-    // bits 2gq of qh[32n + 16(g&1) + t]; sub-block j = 4c + g
-    const int n2 = c >> 1, gq = 2 * (c & 1) + (g >> 1);
-    const uint4 qlv = *reinterpret_cast<const uint4*>(wt + 1024 * (4 * n2 + 2 * (g >> 1) + (g & 1)) + 16 * row);
-    const uint4 qhv = *reinterpret_cast<const uint4*>(wt + 1024 * (8 + 2 * n2 + (g & 1)) + 16 * row);
-    const uint32_t lsh = 4 * (c & 1), hsh = 2 * gq;
-    const uint32_t scd = c == 0 ? sc.x : c == 1 ? sc.y : c == 2 ? sc.z : sc.w;
-    const int scj = (int)(int8_t)((scd >> (8 * g)) & 0xffu);
-    const uint32_t scp = ((uint32_t)scj & 0xffffu) * 0x00010001u;
-    const uint32_t bias = ((uint32_t)(-32 * scj) & 0xffffu) * 0x00010001u;
-    const uint32_t qlw[4] = {qlv.x, qlv.y, qlv.z, qlv.w}, qhw[4] = {qhv.x, qhv.y, qhv.z, qhv.w};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t q = ((qlw[k] >> lsh) & 0x0F0F0F0Fu) | (((qhw[k] >> hsh) & 0x03030303u) << 4);
-      uint32_t hh, ll;
-      q6_split(q, scp, bias, hh, ll);
-      Bh[c][k] = (int)hh;
-      Bl[c][k] = (int)ll;
-    }
-  }
+  for (int c = 0; c < 4; ++c)
+    q6_step_ops(ql[c >> 1], qh[c >> 1], c == 0 ? sc.x : c == 1 ? sc.y : c == 2 ? sc.z : sc.w, c, g, Bh[c], Bl[c]);
+  built();
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     v4i Dh = {0, 0, 0, 0}, Dl = {0, 0, 0, 0};
@@ -258,6 +270,21 @@ __device__ __forceinline__ void q6_block(const uint8_t* wt, const uint8_t* xb, c
       acc[mt][i] += v;
     }
   }
+}
+
+// The same with the weight words in LDS (the packed tile-block wt, the lane's row).
+template <int MT>
+__device__ __forceinline__ void q6_block(const uint8_t* wt, const uint8_t* xb, const float* sb, int row,
+                                         float (&acc)[MT][4]) {
+  const int g = (threadIdx.x & 63) >> 4;
+  uint4 ql[2], qh[2];
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    ql[n] = *reinterpret_cast<const uint4*>(wt + 1024 * (4 * n + 2 * (g >> 1) + (g & 1)) + 16 * row);
+    qh[n] = *reinterpret_cast<const uint4*>(wt + 1024 * (8 + 2 * n + (g & 1)) + 16 * row);
+  }
+  q6_tiles<MT>(ql, qh, *reinterpret_cast<const uint4*>(wt + 1024 * 12 + 16 * row),
+               f16_bits_to_f32(*reinterpret_cast<const uint16_t*>(wt + 1024 * 13 + 2 * row)), xb, sb, acc, [] {});
 }
 
 }  // namespace bb

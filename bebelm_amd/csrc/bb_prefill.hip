@@ -609,11 +609,19 @@ __global__ void __launch_bounds__(512, gemm_waves_per_simd(DT)) k_gemm(const uin
       block(wb1, xb1, sb1);
     }
   };
-  // A tile of MT = 5 that holds at most 64 members computes only its first 4 member tiles (the
-  // others' outputs are not stored), so it costs what a tile of 64 does.
+  // A tile computes only the member tiles that hold members (the others' outputs are not stored), each
+  // count its own straight-line loop: a branch inside the loop spills. Gate/up of 32 experts with
+  // groups of 16 members 55 -> 40 us, of 32 58 -> 50 us, down 26 -> 20 and 27 -> 25 us (Q4_K, hidden
+  // 2048, ff 1792); groups of 48 as before.
   if constexpr (MT == 5) {
     if (__builtin_amdgcn_readfirstlane(ti.cnt) <= 64) sweep(std::integral_constant<int, 4>{});
     else sweep(std::integral_constant<int, 5>{});
+  } else if constexpr (MT == 4 && !MF) {
+    const int cnt = __builtin_amdgcn_readfirstlane(ti.cnt);
+    if (cnt <= 16) sweep(std::integral_constant<int, 1>{});
+    else if (cnt <= 32) sweep(std::integral_constant<int, 2>{});
+    else if (cnt <= 48) sweep(std::integral_constant<int, 3>{});
+    else sweep(std::integral_constant<int, 4>{});
   } else {
     sweep(std::integral_constant<int, MT>{});
   }
@@ -660,6 +668,169 @@ __global__ void __launch_bounds__(512, gemm_waves_per_simd(DT)) k_gemm(const uin
           out[(size_t)outrow[n] * n_out + col] = silu_tab(gate, exptab) * acc[mt][i];
         }
     }
+  } else {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int n = mt * 16 + 4 * g + i;
+        if (outrow[n] < 0) continue;
+        out[(size_t)outrow[n] * n_out + 64 * t64 + 16 * t16 + r] = acc[mt][i];
+      }
+  }
+}
+
+// ---- Q6_K grouped GEMM, weight rows straight into registers --------------------------------------------
+// k_gemm's block and work split (member tile of 16·MT members x two 64-row packed tiles, wave w the 16
+// rows (w & 3) of packed tile w >> 2) with the weights left out of LDS: no wave reads another's rows,
+// so a lane loads its row's words through a buffer resource, two super-blocks ahead (W0, W1), and only
+// the members' activations and scales are staged, one super-block ahead. A Q6_K block of k_gemm fills
+// a CU's LDS with 27 KB of weights a stage and takes 137 registers (one block, two waves a SIMD); this
+// one takes 34 KB and 128, so two blocks share a CU and hide each other's waits. Down of 2048 rows of
+// 1792, 32 experts, k_gemm and here: groups of 16 members 48 and 34 us, 64 members 71 and 49, 128
+// members 104 and 81 (k_gemm in tiles of 128); from 256 members on k_gemm_wide's time (133 us both at
+// 256, 215 at 512). Q4_K rows stay on k_gemm: the same form took 55 to 59 us instead of 55 at groups of
+// 16 (gate/up) and 92 instead of 73 at 64, spilling where k_gemm's operands come from LDS when needed.
+// The copies of a super-block are issued before its weight loads, so waiting for all but the youngest
+// weight loads waits for the copies and for nothing younger.
+struct RowW6 {
+  static constexpr int LOADS = 6;
+  uint4 sc, ql[2], qh[2];
+  uint32_t d;
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, uint32_t row, uint32_t g, uint32_t sb) {
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      ql[n] = buf_load16(r, 16u * row + 1024u * g, sb + 4096u * n);
+      qh[n] = buf_load16(r, 16u * row + 1024u * (g & 1u), sb + 1024u * (8 + 2 * n));
+    }
+    sc = buf_load16(r, 16u * row, sb + 1024u * 12);
+    d = __builtin_amdgcn_raw_buffer_load_b16(r, (int)(1024u * 13 + 2u * row), (int)sb, 0);
+  }
+};
+
+template <int KIND, int MT>
+__global__ void __launch_bounds__(512, 4) k_gemm_r(const uint8_t* __restrict__ wpk, size_t stride_e, int n_in, int K,
+                                                   int n_out, int E, int n_ent, RouteBufs rb, GemmX x,
+                                                   float* __restrict__ out) {
+  constexpr int TB = (int)TB6;
+  constexpr int NBM = 16 * MT;
+  constexpr int XCH = 4 * MT;             // activation copies of 1 KB (four members) a super-block
+  constexpr int SCH = (NBM + 63) / 64;    // scale copies (64 members)
+  constexpr int NC = XCH + SCH, OPS = (NC + 7) / 8;
+  // (every stage an array of its own: reading one then waits for no copy into the other)
+  __shared__ __align__(16) uint8_t xa0[NBM * QK], xa1[NBM * QK];
+  __shared__ __align__(16) float sa0[SCH * 64], sa1[SCH * 64];
+  __shared__ int32_t rowidx[NBM], outrow[NBM];
+  __shared__ int32_t sh[8];
+  __shared__ uint64_t exptab[32];
+  const uint64_t exp_e = KIND == GEMM_GATEUP ? exp_table_entry() : 0;
+  // (blocks to XCDs as in k_gemm with member tiles of 64)
+  const int n_rt = gridDim.y, n_mt = gridDim.x;
+  const int lin = blockIdx.y * n_mt + blockIdx.x;
+  const int xcd = lin & 7, slot = lin >> 3;
+  const int mt_local = slot / n_rt, rt_step = slot % n_rt;
+  const int mtile = mt_local * 8 + xcd;
+  const int rtile = (mt_local & 1) ? n_rt - 1 - rt_step : rt_step;
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nb = n_in / QK;
+  const int k64 = w >> 2, t16 = w & 3, t64 = 2 * rtile + k64;
+  const size_t tile_bytes = (size_t)nb * TB;
+  TileInfo ti;
+  if (!find_tile(rb, E, NBM, mtile, ti, sh)) return;
+  const __amdgpu_buffer_rsrc_t rw = buf_rsrc(
+      wpk + (size_t)__builtin_amdgcn_readfirstlane(ti.e) * stride_e + (size_t)t64 * tile_bytes, (uint32_t)tile_bytes);
+  const uint32_t wrow = (uint32_t)(16 * t16 + r);
+  RowW6 W0, W1;
+  W0.load(rw, wrow, (uint32_t)g, 0);
+  member_rows<KIND>(rb, ti, K, NBM, rowidx, outrow);
+  if (KIND == GEMM_GATEUP && tid < 32) exptab[tid] = exp_e;
+  lds_barrier();
+  const int x_rows = KIND == GEMM_GATEUP ? n_ent / K : n_ent;
+  const __amdgpu_buffer_rsrc_t rx = buf_rsrc(x.q, (uint32_t)x_rows * (uint32_t)n_in);
+  const __amdgpu_buffer_rsrc_t rs = buf_rsrc(x.sx, (uint32_t)x_rows * (uint32_t)nb * 4u);
+  // wave w's copies w, w + 8, ... of a super-block: activations of the tiles that hold members (lane =
+  // member x chunk, swizzled as k_gemm's), then scales
+  const int xch = 4 * ((__builtin_amdgcn_readfirstlane(ti.cnt) + 15) / 16);
+  uint32_t off[OPS];
+#pragma unroll
+  for (int t = 0; t < OPS; ++t) {
+    const int j = w + 8 * t;
+    if (j < XCH) {
+      const int m = 4 * j + (lane >> 4), c = (lane & 15) ^ (m & 15);
+      off[t] = (uint32_t)rowidx[m] * (uint32_t)n_in + 16u * (uint32_t)c;
+    } else {
+      off[t] = (uint32_t)rowidx[min(64 * (j - XCH) + lane, NBM - 1)] * (uint32_t)nb * 4u;
+    }
+  }
+  auto issue = [&](int b, uint8_t* xd, float* sd) {
+#pragma unroll
+    for (int t = 0; t < OPS; ++t) {
+      const int j = w + 8 * t;
+      if (j < XCH) {
+        if (j < xch) buf_dma16(rx, off[t], (uint32_t)(b * QK), xd + j * 1024);
+      } else if (j < NC) {
+        buf_dma4(rs, off[t], (uint32_t)(4 * b), reinterpret_cast<uint8_t*>(sd + 64 * (j - XCH)));
+      }
+    }
+  };
+  issue(0, xa0, sa0);
+  __builtin_amdgcn_sched_barrier(0);
+  W1.load(rw, wrow, (uint32_t)g, (uint32_t)(min(1, nb - 1) * TB));
+  __builtin_amdgcn_sched_barrier(0);
+  const float start = ti.g > 1 ? 0.0f : -0.0f;
+  float acc[MT][4];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[mt][i] = start;
+  auto step = [&](int b, RowW6& W, const uint8_t* xb, const float* sb, uint8_t* xn, float* sn) {
+    constexpr int YOUNG = RowW6::LOADS;  // the weight loads of b + 1 may still be in flight
+    __builtin_amdgcn_s_waitcnt((0x3f70 & ~15) | YOUNG);
+    lds_barrier();  // every wave's copies of b landed, and the stage written next is no longer read
+    if (b + 1 < nb) issue(b + 1, xn, sn);
+    __builtin_amdgcn_sched_barrier(0);
+    q6_tiles<MT>(W.ql, W.qh, W.sc, f16_bits_to_f32(W.d & 0xffff), xb, sb, acc, [&] {
+      __builtin_amdgcn_sched_barrier(0);
+      W.load(rw, wrow, (uint32_t)g, (uint32_t)(min(b + 2, nb - 1) * TB));  // (past the row: its last block again)
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  for (int b = 0; b < nb; b += 2) {
+    step(b, W0, xa0, sa0, xa1, sa1);
+    if (b + 1 >= nb) break;
+    step(b + 1, W1, xa1, sa1, xa0, sa0);
+  }
+  __builtin_amdgcn_s_waitcnt(0x3f70);  // vmcnt(0): nothing in flight past here
+  if constexpr (KIND == GEMM_GATEUP) {
+    // SwiGLU of the wave pair, as k_gemm's: the gate wave takes member tiles mt < MG, the up wave the
+    // rest, each handing the other its values of the other's tiles
+    constexpr int MG = MT - MT / 2;
+    __syncthreads();
+    float* upv = reinterpret_cast<float*>(xa0);  // 4 up waves x MG*4 values x 64 lanes <= sizeof xa0
+    float* gtv = reinterpret_cast<float*>(xa1);  // 4 gate waves x (MT-MG)*4 values x 64 lanes
+    const int pair = k64 * 2 + (t16 & 1);
+    const bool up = t16 >= 2;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (up && mt < MG) upv[(pair * (4 * MG) + mt * 4 + i) * 64 + lane] = acc[mt][i];
+        if (!up && mt >= MG) gtv[(pair * (4 * (MT - MG)) + (mt - MG) * 4 + i) * 64 + lane] = acc[mt][i];
+      }
+    __syncthreads();
+    const int col = 32 * t64 + 16 * (t16 & 1) + r;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (up != (mt >= MG)) continue;
+        const int n = mt * 16 + 4 * g + i;
+        if (outrow[n] < 0) continue;
+        const float gate = up ? gtv[(pair * (4 * (MT - MG)) + (mt - MG) * 4 + i) * 64 + lane] : acc[mt][i];
+        const float upval = up ? acc[mt][i] : upv[(pair * (4 * MG) + mt * 4 + i) * 64 + lane];
+        out[(size_t)outrow[n] * n_out + col] = silu_tab(gate, exptab) * upval;
+      }
   } else {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
@@ -1064,10 +1235,8 @@ __global__ void __launch_bounds__(64 * WIDE_WAVES, 2) k_gemm_wide(const uint8_t*
 }
 
 // Member tile (in units of 16 members): 16 for decode-sized batches (these tiles take their
-// grouping from the selections), else 64; Q6_K rows take 128 when the groups fill such tiles
-// on average. (A Q4_K block of 64 members leaves room for two blocks per CU, which beat one
-// block of 128 members: 483 vs 554 µs for config 4's gate/up. A Q6_K block of 64 members
-// still fills a CU's LDS alone.)
+// grouping from the selections), else 64. (A Q4_K block of 64 members leaves room for two blocks per
+// CU, which beat one block of 128 members: 483 vs 554 µs for config 4's gate/up.)
 int gemm_member_tiles(int n_ent, int E) { return n_ent >= 16 * E ? 4 : 1; }
 
 bool gateup16_applies(int dtype, int T, int H, int F, int E, int K, bool act_q8) {
@@ -1078,8 +1247,8 @@ bool gateup16_applies(int dtype, int T, int H, int F, int E, int K, bool act_q8)
 
 bool down16_applies(int dtype, int T, int H, int F, int E, int K) {
   const int n_ent = T * K;
-  return dtype == DT_Q4_K && gemm_member_tiles(n_ent, E) == 1 && T <= 16 && n_ent <= 64 && H % 256 == 0 &&
-         F % QK == 0 && F / QK >= 1 && F / QK <= 8;
+  return (dtype == DT_Q4_K || dtype == DT_Q6_K) && gemm_member_tiles(n_ent, E) == 1 && T <= 16 && n_ent <= 64 &&
+         H % 256 == 0 && F % QK == 0 && F / QK >= 1 && F / QK <= 8;
 }
 
 // ---- Q4_K gate/up of decode batches (at most 16 tokens): weight rows straight into registers -------
@@ -1288,7 +1457,7 @@ __global__ void __launch_bounds__(64 * GU16_WAVES, 4) k_gateup16(const uint8_t* 
   }
 }
 
-// ---- Q4_K down of decode batches (at most 16 members per expert): weight rows into registers ------
+// ---- down of decode batches (at most 16 members per expert): weight rows into registers -------------
 // k_gateup16's form for the down GEMM. Work unit = one expert x 16 output rows (a quarter of a
 // 64-row packed tile); block = GU16_WAVES waves on the expert's rows 256j..256j+255, H/256 blocks
 // per expert, expert-major. A token chooses an expert at most once, so an expert of a batch of at
@@ -1297,14 +1466,62 @@ __global__ void __launch_bounds__(64 * GU16_WAVES, 4) k_gateup16(const uint8_t* 
 // block requests its first weights from its id, reads the selections, copies its members' act
 // rows (all NB super-blocks, XOR-swizzled chunks as k_gemm stages them) and their scales into LDS,
 // and streams the rest of its weights through the register ring while it computes. The integer
-// sums and the f32 epilogue are q4_block's (gu16_tile), from +0.0 (-0.0 for an expert with one
+// sums and the f32 epilogue are q4_block's or q6_block's, from +0.0 (-0.0 for an expert with one
 // member, as k_gemm); member m's outputs go to the slot row of its entry.
-template <int NB>
+// Q6_K rows (the same blocks, q6_block's two passes) are bound by their operand build, about 250
+// vector instructions a wave and super-block against 95: config 2's layer with Q6_K down 30.7 us on
+// k_gemm, 22.2 here (16 tokens).
+template <int DT>
+struct Dn16H;
+template <>
+struct Dn16H<DT_Q4_K> : Gu16H {
+  static constexpr int LOADS = 3;
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, uint32_t row, uint32_t g, uint32_t sb) {
+    gu16_load(*this, r, 16u * row, 1024u * (1 + 2 * g), sb);
+  }
+  __device__ __forceinline__ void tile(const uint8_t* xb, const float* sb, float (&acc)[4]) const {
+    gu16_tile(h, q0, q1, xb, sb, acc);
+  }
+};
+template <>
+struct Dn16H<DT_Q6_K> {
+  static constexpr int LOADS = 6;
+  uint4 sc, ql[2], qh[2];
+  uint32_t d;
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, uint32_t row, uint32_t g, uint32_t sb) {
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      ql[n] = buf_load16nt(r, 16u * row + 1024u * g, sb + 4096u * n);
+      qh[n] = buf_load16nt(r, 16u * row + 1024u * (g & 1u), sb + 1024u * (8 + 2 * n));
+    }
+    sc = buf_load16nt(r, 16u * row, sb + 1024u * 12);
+    d = __builtin_amdgcn_raw_buffer_load_b16(r, (int)(1024u * 13 + 2u * row), (int)sb, CPOL_NT);
+  }
+  __device__ __forceinline__ void tile(const uint8_t* xb, const float* sb, float (&acc)[4]) const {
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    v4i Dh = {0, 0, 0, 0}, Dl = {0, 0, 0, 0};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const v4i ax = read_x16(xb, r, 4 * c + g);
+      v4i Bh, Bl;
+      q6_step_ops(ql[c >> 1], qh[c >> 1], c == 0 ? sc.x : c == 1 ? sc.y : c == 2 ? sc.z : sc.w, c, g, Bh, Bl);
+      Dh = __builtin_amdgcn_mfma_i32_16x16x64_i8(ax, Bh, Dh, 0, 0, 0);
+      Dl = __builtin_amdgcn_mfma_i32_16x16x64_i8(ax, Bl, Dl, 0, 0, 0);
+    }
+    const float dd = f16_bits_to_f32(d & 0xffff);
+    const float4 sx4 = *reinterpret_cast<const float4*>(sb + 4 * g);
+    const float sxv[4] = {sx4.x, sx4.y, sx4.z, sx4.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] += sxv[i] * (dd * (float)(64 * Dh[i] + Dl[i]));
+  }
+};
+
+template <int DT, int NB>
 __global__ void __launch_bounds__(64 * GU16_WAVES, 4) k_down16(const uint8_t* __restrict__ wpk, size_t stride_e,
                                                               int n_out, int n_ent,
                                                               const int32_t* __restrict__ sel, GemmX x,
                                                               float* __restrict__ out, int act_pad) {
-  constexpr int TB = (int)TB4;
+  constexpr int TB = GemmTraits<DT>::TB;
   constexpr int XB = 16 * QK;  // one super-block of 16 members' quants
   constexpr int NW = GU16_WAVES;
   constexpr int NC = (4 * NB + NW - 1) / NW;  // activation copies per wave
@@ -1345,15 +1562,16 @@ __global__ void __launch_bounds__(64 * GU16_WAVES, 4) k_down16(const uint8_t* __
   const __amdgpu_buffer_rsrc_t rsrc = buf_rsrc(wpk + (size_t)e * stride_e + (size_t)t64 * tile_bytes,
                                                (uint32_t)tile_bytes);
   // half h = super-block h of the wave's 16 rows
-  const uint32_t og = 16u * (uint32_t)(16 * t16 + r), oq = 1024u * (uint32_t)(1 + 2 * g);
+  const uint32_t wrow = (uint32_t)(16 * t16 + r);
   constexpr int AHEAD = DN16_SLOTS - 1;
-  auto half_load = [&](Gu16H& v, int h) { gu16_load(v, rsrc, og, oq, (uint32_t)(h * TB)); };
-  Gu16H wr[DN16_SLOTS];
+  using H16 = Dn16H<DT>;
+  auto half_load = [&](H16& v, int h) { v.load(rsrc, wrow, (uint32_t)g, (uint32_t)(h * TB)); };
+  H16 wr[DN16_SLOTS];
   half_load(wr[0], 0);
   __builtin_amdgcn_sched_barrier(0);
   // this wave's selection copy (and act copies) landed (the weight loads issued after them may
   // still be in flight)
-  constexpr int WS = 3;
+  constexpr int WS = H16::LOADS;
   __builtin_amdgcn_s_waitcnt(0x3f70 | (WS & 15) | ((WS >> 4) << 14));
   // the expert's entries (entry i on lane i) and the entries of smaller expert ids (the first
   // group position of its members)
@@ -1370,7 +1588,7 @@ __global__ void __launch_bounds__(64 * GU16_WAVES, 4) k_down16(const uint8_t* __
   for (int h = 1; h <= NL; ++h) half_load(wr[h], h);
   __builtin_amdgcn_sched_barrier(0);
   // this wave's copies landed (the weight loads issued after them may still be in flight)
-  constexpr int WL = 3 * NL;
+  constexpr int WL = H16::LOADS * NL;
   __builtin_amdgcn_s_waitcnt(0x3f70 | (WL & 15) | ((WL >> 4) << 14));
   lds_barrier();
   const float start = cnt > 1 ? 0.0f : -0.0f;
@@ -1380,8 +1598,7 @@ __global__ void __launch_bounds__(64 * GU16_WAVES, 4) k_down16(const uint8_t* __
     // the slot half h-1 used takes half h+AHEAD
     if (h + AHEAD < NB) half_load(wr[(h + AHEAD) % DN16_SLOTS], h + AHEAD);
     __builtin_amdgcn_sched_barrier(0);
-    const Gu16H& cur = wr[h % DN16_SLOTS];
-    gu16_tile(cur.h, cur.q0, cur.q1, xs + h * XB, sxs + 16 * h, acc);
+    wr[h % DN16_SLOTS].tile(xs + h * XB, sxs + 16 * h, acc);
 #pragma unroll
     for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(acc[i]));
     __builtin_amdgcn_sched_barrier(0);
@@ -1422,7 +1639,7 @@ static hipError_t launch_gemm(hipStream_t s, const uint8_t* w, size_t stride_e, 
       return hipGetLastError();
     }
   }
-  int mt = DT == DT_Q6_K && n_ent >= 128 * E ? 8 : gemm_member_tiles(n_ent, E);
+  int mt = gemm_member_tiles(n_ent, E);
   // Q4_K groups of 48+ members on average: member tiles of 80 (groups of 64 +- 8 then take one
   // tile where tiles of 64 often took a second one nearly empty); one group of known size takes
   // the tile that pads it less
@@ -1446,13 +1663,13 @@ static hipError_t launch_gemm(hipStream_t s, const uint8_t* w, size_t stride_e, 
       return hipGetLastError();
     }
   }
-  if constexpr (DT == DT_Q4_K && KIND == GEMM_DOWN) {
+  if constexpr (KIND == GEMM_DOWN) {
     // decode batches of at most 16 tokens (an expert then has at most 16 members): k_down16
     if (rb.sel && down16_applies(DT, T, n_out, n_in, E, K)) {
       const dim3 grid(E * (n_out / 256)), block(64 * GU16_WAVES);
       switch (n_in / QK) {
 #define BB_DOWN16(nb) \
-  case nb: BB_LAUNCH(k_down16<nb>, grid, block, 0, s, w, stride_e, n_out, n_ent, rb.sel, x, out, (int)act_pad); break;
+  case nb: BB_LAUNCH((k_down16<DT, nb>), grid, block, 0, s, w, stride_e, n_out, n_ent, rb.sel, x, out, (int)act_pad); break;
         BB_DOWN16(1) BB_DOWN16(2) BB_DOWN16(3) BB_DOWN16(4) BB_DOWN16(5) BB_DOWN16(6) BB_DOWN16(7) BB_DOWN16(8)
 #undef BB_DOWN16
       }
@@ -1468,12 +1685,14 @@ static hipError_t launch_gemm(hipStream_t s, const uint8_t* w, size_t stride_e, 
   const uint64_t x_rows = KIND == GEMM_GATEUP ? (uint64_t)T : (uint64_t)n_ent;
   const uint64_t tile2 = 2ull * (uint64_t)(n_in / QK) * (uint64_t)GemmTraits<DT>::TB;
   const bool buf = x_rows * (uint64_t)n_in < (1ull << 31) && tile2 < (1ull << 31);
-  if (DT == DT_Q6_K && mt == 8 && buf)
-    BB_LAUNCH((k_gemm<DT_Q6_K, KIND, 8, true>), grid, dim3(512), 0, s, w, stride_e, n_in, K, n_out, E, n_ent, rb, x,
-              out);
-  else if (DT == DT_Q6_K && mt == 8)
-    BB_LAUNCH((k_gemm<DT_Q6_K, KIND, 8>), grid, dim3(512), 0, s, w, stride_e, n_in, K, n_out, E, n_ent, rb, x, out);
-  else if (DT == DT_Q4_K && mt == 5 && buf)
+  // (k_gemm_r: buffer offsets only; inputs past them keep k_gemm)
+  if constexpr (DT == DT_Q6_K) {
+    if (mt == 4 && buf) {
+      BB_LAUNCH((k_gemm_r<KIND, 4>), grid, dim3(512), 0, s, w, stride_e, n_in, K, n_out, E, n_ent, rb, x, out);
+      return hipGetLastError();
+    }
+  }
+  if (DT == DT_Q4_K && mt == 5 && buf)
     BB_LAUNCH((k_gemm<DT_Q4_K, KIND, 5, true>), grid, dim3(512), 0, s, w, stride_e, n_in, K, n_out, E, n_ent, rb, x,
               out);
   else if (DT == DT_Q4_K && mt == 5)
@@ -1481,8 +1700,8 @@ static hipError_t launch_gemm(hipStream_t s, const uint8_t* w, size_t stride_e, 
   else if (DT == DT_Q4_K && mt == 4 && buf && ms)
     BB_LAUNCH((k_gemm<DT_Q4_K, KIND, 4, true, true>), grid, dim3(512), 0, s, w, stride_e, n_in, K, n_out, E, n_ent,
               rb, x, out);
-  else if (mt == 4 && buf)
-    BB_LAUNCH((k_gemm<DT, KIND, 4, true>), grid, dim3(512), 0, s, w, stride_e, n_in, K, n_out, E, n_ent, rb, x, out);
+  else if (DT == DT_Q4_K && mt == 4 && buf)
+    BB_LAUNCH((k_gemm<DT_Q4_K, KIND, 4, true>), grid, dim3(512), 0, s, w, stride_e, n_in, K, n_out, E, n_ent, rb, x, out);
   else if (mt == 4)
     BB_LAUNCH((k_gemm<DT, KIND, 4>), grid, dim3(512), 0, s, w, stride_e, n_in, K, n_out, E, n_ent, rb, x, out);
   else
@@ -1507,7 +1726,8 @@ hipError_t launch_gemm_down(hipStream_t s, int dtype, const uint8_t* dn, size_t 
   if (dtype == DT_Q4_K)
     return launch_gemm<DT_Q4_K, GEMM_DOWN>(s, dn, stride_dn, T, F, H, H / 64, E, K, rb, x, slots, nullptr, nullptr,
                                            nullptr, act_pad);
-  return launch_gemm<DT_Q6_K, GEMM_DOWN>(s, dn, stride_dn, T, F, H, H / 64, E, K, rb, x, slots);
+  return launch_gemm<DT_Q6_K, GEMM_DOWN>(s, dn, stride_dn, T, F, H, H / 64, E, K, rb, x, slots, nullptr, nullptr,
+                                         nullptr, act_pad);
 }
 
 // ---- one group of T tokens (dense projections on the grouped GEMM) ----------------------------------

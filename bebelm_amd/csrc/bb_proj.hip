@@ -77,22 +77,8 @@ __device__ __forceinline__ void proj_build(const ProjW<DT_Q6_K>& w, int g, ProjB
   o.d = f16_bits_to_f32(w.d & 0xffff);
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
-    const int gq = 2 * (c & 1) + (g >> 1);
-    const uint4 qlv = w.ql[c >> 1], qhv = w.qh[c >> 1];
-    const uint32_t lsh = 4 * (c & 1), hsh = 2 * gq;
-    const uint32_t scd = c == 0 ? w.sc.x : c == 1 ? w.sc.y : c == 2 ? w.sc.z : w.sc.w;
-    const int scj = (int)(int8_t)((scd >> (8 * g)) & 0xffu);
-    const uint32_t scp = ((uint32_t)scj & 0xffffu) * 0x00010001u;
-    const uint32_t bias = ((uint32_t)(-32 * scj) & 0xffffu) * 0x00010001u;
-    const uint32_t qlw[4] = {qlv.x, qlv.y, qlv.z, qlv.w}, qhw[4] = {qhv.x, qhv.y, qhv.z, qhv.w};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t q = ((qlw[k] >> lsh) & 0x0F0F0F0Fu) | (((qhw[k] >> hsh) & 0x03030303u) << 4);
-      uint32_t hh, ll;
-      q6_split(q, scp, bias, hh, ll);
-      o.hi[c][k] = (int)hh;
-      o.lo[c][k] = (int)ll;
-    }
+    q6_step_ops(w.ql[c >> 1], w.qh[c >> 1], c == 0 ? w.sc.x : c == 1 ? w.sc.y : c == 2 ? w.sc.z : w.sc.w, c, g, o.hi[c],
+                o.lo[c]);
   }
 }
 

@@ -6,8 +6,8 @@ rows, so that every address a launch can touch is checked against the size of th
 belongs to on the CPU, for any routing, before a shape ever runs on the GPU.
 
 What is modelled (per block of the launch the host code in launch_gemm would make):
-  * the launch choice (k_gateup16 / k_gemm with member tiles of 16, 64, 80 or 128 / k_gemm_wide)
-    and its grid;
+  * the launch choice (k_gateup16 / k_gemm with member tiles of 16, 64 or 80 / k_gemm_r, the
+    Q6_K form with k_gemm's tiles of 64, rows and copies / k_gemm_wide) and its grid;
   * the block -> (member tile, row tile) mapping, including the XCD-aware order;
   * the member tile: expert, first member, count, group base (find_tile, expert_tile,
     hit_expert_tile, find_wide_tile), and the member rows and output rows (member_rows,
@@ -97,7 +97,7 @@ def launch_choice(s):
     n_ent, E = s.n_ent, s.E
     if s.dt == Q6_K and s.kind == DOWN and n_ent >= WIDE_MIN_AVG * E and n_ent * s.n_in < (1 << 31):
         return ("wide", (n_ent // WIDE_NB + (WIDE_LOG + 1) * E + 7) // 8 * 8)
-    mt = 8 if s.dt == Q6_K and n_ent >= 128 * E else (4 if n_ent >= 16 * E else 1)
+    mt = 4 if n_ent >= 16 * E else 1
     if s.dt == Q4_K and mt == 4 and n_ent >= 48 * E and not reads_ms(s):
         mt = 5 if E > 1 or (n_ent + 79) // 80 * 5 < (n_ent + 63) // 64 * 4 else 4
     if (s.dt == Q4_K and s.kind == GATEUP and mt == 1 and s.quant and s.T <= 16 and n_ent <= 64 and E <= 32
