@@ -693,18 +693,23 @@ __global__ void __launch_bounds__(512, gemm_waves_per_simd(DT)) k_gemm(const uin
 // 16 (gate/up) and 92 instead of 73 at 64, spilling where k_gemm's operands come from LDS when needed.
 // The copies of a super-block are issued before its weight loads, so waiting for all but the youngest
 // weight loads waits for the copies and for nothing younger.
+// (NT: the words are read once)
+template <bool NT>
 struct RowW6 {
   static constexpr int LOADS = 6;
   uint4 sc, ql[2], qh[2];
   uint32_t d;
+  static __device__ __forceinline__ uint4 load16(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t sb) {
+    return NT ? buf_load16nt(r, off, sb) : buf_load16(r, off, sb);
+  }
   __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, uint32_t row, uint32_t g, uint32_t sb) {
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
-      ql[n] = buf_load16(r, 16u * row + 1024u * g, sb + 4096u * n);
-      qh[n] = buf_load16(r, 16u * row + 1024u * (g & 1u), sb + 1024u * (8 + 2 * n));
+      ql[n] = load16(r, 16u * row + 1024u * g, sb + 4096u * n);
+      qh[n] = load16(r, 16u * row + 1024u * (g & 1u), sb + 1024u * (8 + 2 * n));
     }
-    sc = buf_load16(r, 16u * row, sb + 1024u * 12);
-    d = __builtin_amdgcn_raw_buffer_load_b16(r, (int)(1024u * 13 + 2u * row), (int)sb, 0);
+    sc = load16(r, 16u * row, sb + 1024u * 12);
+    d = __builtin_amdgcn_raw_buffer_load_b16(r, (int)(1024u * 13 + 2u * row), (int)sb, NT ? CPOL_NT : 0);
   }
 };
 
@@ -741,7 +746,8 @@ __global__ void __launch_bounds__(512, 4) k_gemm_r(const uint8_t* __restrict__ w
   const __amdgpu_buffer_rsrc_t rw = buf_rsrc(
       wpk + (size_t)__builtin_amdgcn_readfirstlane(ti.e) * stride_e + (size_t)t64 * tile_bytes, (uint32_t)tile_bytes);
   const uint32_t wrow = (uint32_t)(16 * t16 + r);
-  RowW6 W0, W1;
+  using W6 = RowW6<false>;
+  W6 W0, W1;
   W0.load(rw, wrow, (uint32_t)g, 0);
   member_rows<KIND>(rb, ti, K, NBM, rowidx, outrow);
   if (KIND == GEMM_GATEUP && tid < 32) exptab[tid] = exp_e;
@@ -784,8 +790,8 @@ __global__ void __launch_bounds__(512, 4) k_gemm_r(const uint8_t* __restrict__ w
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[mt][i] = start;
-  auto step = [&](int b, RowW6& W, const uint8_t* xb, const float* sb, uint8_t* xn, float* sn) {
-    constexpr int YOUNG = RowW6::LOADS;  // the weight loads of b + 1 may still be in flight
+  auto step = [&](int b, W6& W, const uint8_t* xb, const float* sb, uint8_t* xn, float* sn) {
+    constexpr int YOUNG = W6::LOADS;  // the weight loads of b + 1 may still be in flight
     __builtin_amdgcn_s_waitcnt((0x3f70 & ~15) | YOUNG);
     lds_barrier();  // every wave's copies of b landed, and the stage written next is no longer read
     if (b + 1 < nb) issue(b + 1, xn, sn);
@@ -1614,6 +1620,231 @@ __global__ void __launch_bounds__(64 * GU16_WAVES, 4) k_down16(const uint8_t* __
   }
 }
 
+// ---- batches between the two: up to 32 members of an expert, weight rows into registers --------------
+// The form of k_gateup16 and k_down16 (16 waves on an expert's outputs 256j..256j+255, a wave's
+// weight rows straight into its registers) for the batches above 16 tokens whose groups still average
+// fewer than 16: the members come from the selections (n_ent < 16·E <= 512 entries), tile u of an
+// expert is its members 32u..32u+31 (first the experts' first tiles, whose expert is known from the
+// block's id, then the others), and all super-blocks of the tile's Q8 rows stay in LDS (64 KB), so the weights stream with no barrier and no copy beside them. What bounds it is the
+// operand build, about 95 (Q4_K) or 250 (Q6_K) vector instructions a wave and super-block, which the
+// member tiles share (a third and a fourth spill). Gate/up takes the gate and the up rows of a wave's 16 outputs in turn, applies
+// SwiGLU in the lane that holds both, and quantises the act rows as k_gateup16 does.
+// k_gemm in member tiles of 16 staged the weights through LDS beside the activations and built the
+// operands anew for every 16 members: config 2's layer, gate/up with the act rows' Q8 (a launch of its
+// own there) 39 -> 28 us at 49 tokens and 57 -> 42 at 127, down Q4_K 17 -> 16 and 25 -> 22, Q6_K 32 ->
+// 26 and 51 -> 31.
+constexpr int MID_BN = 32;               // members of a block
+constexpr int MID_NB = 8;                // super-blocks of an input row
+// Fewer blocks (E x outputs / 256) leave CUs idle where k_gemm's of 64 or 128 rows fill them: down of
+// 2048 outputs, Q4_K, 64 blocks 12 us on k_gemm and 17 here, 128 15.3 and 18.7, 160 20.1 and 19.4, 256 17
+// and 16; gate/up with its Q8, 56 blocks 23 and 36, 140 36 and 37, 224 39 and 28.
+constexpr int MID_MIN_BLOCKS = 160;
+
+// A lane's words of one 16-row tile and super-block (q4_tiles' and q6_tiles' operands).
+struct RowW4 {
+  static constexpr int LOADS = 3;
+  uint4 h, q[2];
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, uint32_t row, uint32_t g, uint32_t sb) {
+    h = buf_load16nt(r, 16u * row, sb);
+    q[0] = buf_load16nt(r, 16u * row + 1024u * (1u + 2u * g), sb);
+    q[1] = buf_load16nt(r, 16u * row + 1024u * (2u + 2u * g), sb);
+  }
+};
+
+template <int MT, class Built>
+__device__ __forceinline__ void row_tiles(const RowW4& w, const uint8_t* xb, const float* sb, float (&acc)[MT][4],
+                                          Built&& built) {
+  q4_tiles<MT>(w.h, w.q, xb, sb, nullptr, acc, built);
+}
+template <int MT, class Built>
+__device__ __forceinline__ void row_tiles(const RowW6<true>& w, const uint8_t* xb, const float* sb, float (&acc)[MT][4],
+                                          Built&& built) {
+  q6_tiles<MT>(w.ql, w.qh, w.sc, f16_bits_to_f32(w.d & 0xffff), xb, sb, acc, built);
+}
+
+template <int DT, int KIND>
+__global__ void __launch_bounds__(64 * GU16_WAVES, 4) k_gemm_mid(const uint8_t* __restrict__ wpk, size_t stride_e,
+                                                                int nb, int n_out, int E, int K, int n_ent,
+                                                                const int32_t* __restrict__ sel, GemmX x,
+                                                                float* __restrict__ out, int8_t* __restrict__ aq,
+                                                                float* __restrict__ aq_sx) {
+  constexpr int TB = GemmTraits<DT>::TB;
+  constexpr int NW = GU16_WAVES;
+  constexpr int HALVES = KIND == GEMM_GATEUP ? 2 : 1;  // row tiles of a wave
+  using W = std::conditional_t<DT == DT_Q4_K, RowW4, RowW6<true>>;
+  __shared__ __align__(16) uint8_t xs[MID_NB * MID_BN * QK];  // [super-block][member], chunks swizzled
+  __shared__ __align__(16) float sxs[MID_NB * MID_BN];        // [super-block][member]
+  __shared__ int32_t ents[MID_BN];                            // the tile's entries
+  __shared__ int32_t eqc[8], ltc[8], cnts[32];
+  __shared__ uint64_t exptab[32];
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int bpe = n_out / (16 * NW);  // blocks of an expert's outputs
+  const int j = blockIdx.x % bpe;
+  const int o = j * NW + w;           // the wave's 16 outputs
+  // entries 64k..64k+63 are wave k's (n_ent <= 512)
+  const int sv = tid < n_ent ? sel[tid] : -1;
+  int e = blockIdx.x / bpe, m0 = 0;
+  if (e >= E) {
+    // the (e - E)-th further tile of the experts that have more than MID_BN members
+    if (tid < 32) cnts[tid] = 0;
+    lds_barrier();
+    if (sv >= 0) atomicAdd(&cnts[sv], 1);
+    lds_barrier();
+    int u = e - E;
+    const int c = lane < 32 ? cnts[lane] : 0;
+    uint32_t big = (uint32_t)__ballot(c > MID_BN);  // the same in every wave
+    for (;; big &= big - 1) {
+      if (!big) return;
+      e = __builtin_ctz(big);
+      const int more = (__builtin_amdgcn_readlane(c, e) - 1) / MID_BN;
+      if (u < more) break;
+      u -= more;
+    }
+    m0 = MID_BN * (u + 1);
+  }
+  e = __builtin_amdgcn_readfirstlane(e);
+  m0 = __builtin_amdgcn_readfirstlane(m0);
+  const uint64_t exp_e = KIND == GEMM_GATEUP ? exp_table_entry() : 0;
+  const int t64 = KIND == GEMM_GATEUP ? o >> 1 : o >> 2;
+  const uint32_t wrow = (uint32_t)(16 * (KIND == GEMM_GATEUP ? o & 1 : o & 3) + r);
+  const size_t tile_bytes = (size_t)nb * TB;
+  const __amdgpu_buffer_rsrc_t rsrc = buf_rsrc(wpk + (size_t)e * stride_e + (size_t)t64 * tile_bytes,
+                                               (uint32_t)tile_bytes);
+  // step t = super-block t / HALVES of row tile t % HALVES (gate rows, then the up rows 32 below)
+  const int n_step = HALVES * nb;
+  W w0, w1;
+  auto load = [&](W& v, int t) {
+    v.load(rsrc, HALVES == 2 ? wrow + 32u * (uint32_t)(t & 1) : wrow, (uint32_t)g, (uint32_t)(t / HALVES * TB));
+  };
+  __builtin_amdgcn_sched_barrier(0);
+  load(w0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  const unsigned long long me = __ballot(sv == e), lt = __ballot(sv >= 0 && sv < e);
+  if (w < 8 && lane == 0) {
+    eqc[w] = __popcll(me);
+    ltc[w] = __popcll(lt);
+  }
+  if (KIND == GEMM_GATEUP && tid < 32) exptab[tid] = exp_e;
+  lds_barrier();
+  int cnt = 0, first = 0, before = 0;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    cnt += eqc[k];
+    first += ltc[k];
+    before += k < w ? eqc[k] : 0;
+  }
+  cnt = __builtin_amdgcn_readfirstlane(cnt);
+  first = __builtin_amdgcn_readfirstlane(first) + m0;  // the tile's first group position
+  const int n = __builtin_amdgcn_readfirstlane(min(MID_BN, cnt - m0));
+  if (n <= 0) {
+    __builtin_amdgcn_s_waitcnt(0x3f70);  // vmcnt(0)
+    return;
+  }
+  if (sv == e) {
+    const int k = before + __popcll(me & ((1ull << lane) - 1ull)) - m0;
+    if (k >= 0 && k < MID_BN) ents[k] = tid;
+  }
+  if (KIND == GEMM_GATEUP) lds_barrier();  // (down copies by group position)
+  // copies of 1 KB (four members' 256 quants of a super-block), then two super-blocks' scales a wave;
+  // members past the last repeat its row
+  const int xlog = n > 16 ? 3 : 2;  // log2 of a super-block's copies
+  auto x_row = [&](int m) {
+    const int k = min(m, n - 1);
+    return (size_t)(KIND == GEMM_GATEUP ? ents[k] / K : first + k);
+  };
+  for (int u = w; u < nb << xlog; u += NW) {
+    const int b = u >> xlog, i = u & ((1 << xlog) - 1), m = 4 * i + (lane >> 4);
+    lds_dma16(reinterpret_cast<const uint8_t*>(x.q) + x_row(m) * (size_t)(nb * QK) + b * QK + 16 * ((lane & 15) ^ (m & 15)),
+              xs + b * (MID_BN * QK) + i * 1024);
+  }
+  if (w < (nb + 1) / 2) {  // scales of super-blocks 2w and 2w + 1
+    const int b = min(2 * w + (lane >> 5), nb - 1);
+    lds_dma4(reinterpret_cast<const uint8_t*>(x.sx + x_row(lane & 31) * (size_t)nb + b),
+             reinterpret_cast<uint8_t*>(sxs + 2 * MID_BN * w));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  load(w1, min(1, n_step - 1));
+  __builtin_amdgcn_sched_barrier(0);
+  // this wave's copies landed (the weight loads issued after them may still be in flight)
+  __builtin_amdgcn_s_waitcnt((0x3f70 & ~15) | W::LOADS);
+  lds_barrier();
+  const float start = cnt > 1 ? 0.0f : -0.0f;
+  // the first M member tiles, each count its own loop (a branch inside one spills)
+  auto body = [&](auto mc) {
+    constexpr int M = decltype(mc)::value;
+    float acc[HALVES][M][4];
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+      for (int mt = 0; mt < M; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[h][mt][i] = start;
+    auto step = [&](int t, float(&am)[M][4], W& v) {
+      const int b = t / HALVES;
+      row_tiles<M>(v, xs + b * (MID_BN * QK), sxs + MID_BN * b, am, [&] {
+        __builtin_amdgcn_sched_barrier(0);
+        load(v, min(t + 2, n_step - HALVES + (t & (HALVES - 1))));  // (past the row: its last block again)
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    };
+    for (int t = 0; t < n_step; t += 2) {
+      step(t, acc[0], w0);
+      if (HALVES == 1 && t + 1 >= n_step) break;
+      step(t + 1, acc[HALVES - 1], w1);
+    }
+    if constexpr (KIND == GEMM_GATEUP) {
+      // the block's 256 outputs of every member, over the activations
+      float* const actv = reinterpret_cast<float*>(xs);
+      lds_barrier();  // the last super-block has been read
+#pragma unroll
+      for (int mt = 0; mt < M; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          actv[(16 * mt + 4 * g + i) * QK + 16 * w + r] = silu_tab(acc[0][mt][i], exptab) * acc[HALVES - 1][mt][i];
+    } else {
+#pragma unroll
+      for (int mt = 0; mt < M; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int m = 16 * mt + 4 * g + i;
+          if (m < n) out[(size_t)ents[m] * n_out + 16 * o + r] = acc[0][mt][i];
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0x3f70);  // vmcnt(0): nothing in flight past here
+    if constexpr (KIND == GEMM_GATEUP) {
+      lds_barrier();
+      // wave w quantises members w, w + 16
+      for (int m = w; m < n; m += NW) {
+        const float4 v = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(xs) + m * QK + 4 * lane);
+        const size_t row = (size_t)(first + m);
+        wave_quantize_xq(v, aq + row * n_out + j * QK, aq_sx + row * (n_out / QK) + j, nullptr);
+      }
+    }
+  };
+  if (n <= 16) {
+    body(std::integral_constant<int, 1>{});
+    return;
+  }
+  body(std::integral_constant<int, 2>{});
+}
+
+// (n_out: the outputs of an expert, F for gate/up and H for down)
+static bool mid_applies(int n_ent, int n_in, int n_out, int E) {
+  return gemm_member_tiles(n_ent, E) == 1 && E <= 32 && n_out % QK == 0 && n_in / QK <= MID_NB &&
+         E * (n_out / QK) >= MID_MIN_BLOCKS;
+}
+
+template <int DT, int KIND>
+static hipError_t launch_mid(hipStream_t s, const uint8_t* w, size_t stride_e, int T, int n_in, int n_out, int E, int K,
+                             const int32_t* sel, GemmX x, float* out, int8_t* aq, float* aq_sx) {
+  // an expert's first tile each, and the further tiles: c members (at most T) give (c - 1) / MID_BN
+  const int n_tile = T <= MID_BN ? E : E + (T * K - 1) / MID_BN;
+  BB_LAUNCH((k_gemm_mid<DT, KIND>), dim3((unsigned)(n_tile * (n_out / QK))), dim3(64 * GU16_WAVES), 0, s, w, stride_e,
+            n_in / QK, n_out, E, K, T * K, sel, x, out, aq, aq_sx);
+  return hipGetLastError();
+}
+
 // Q6_K down GEMMs whose groups hold this many members on average take k_gemm_wide (blocks of up
 // to 256 members). For config 4 (4096 tokens, Zipf-skewed groups) it runs the Q6_K down GEMM in
 // 228 µs against k_gemm's 274; the Q4_K gate/up GEMM, whose 3-pass epilogue and operand build
@@ -1662,6 +1893,10 @@ static hipError_t launch_gemm(hipStream_t s, const uint8_t* w, size_t stride_e, 
       if (quantized) *quantized = true;
       return hipGetLastError();
     }
+    if (rb.sel && aq && mid_applies(n_ent, n_in, n_out, E)) {
+      if (quantized) *quantized = true;
+      return launch_mid<DT, KIND>(s, w, stride_e, T, n_in, n_out, E, K, rb.sel, x, nullptr, aq, aq_sx);
+    }
   }
   if constexpr (KIND == GEMM_DOWN) {
     // decode batches of at most 16 tokens (an expert then has at most 16 members): k_down16
@@ -1675,6 +1910,8 @@ static hipError_t launch_gemm(hipStream_t s, const uint8_t* w, size_t stride_e, 
       }
       return hipGetLastError();
     }
+    if (rb.sel && mid_applies(n_ent, n_in, n_out, E))
+      return launch_mid<DT, KIND>(s, w, stride_e, T, n_in, n_out, E, K, rb.sel, x, out, nullptr, nullptr);
   }
   const int bn = 16 * mt;
   // enough member tiles: with tiles of 16, ceil(T/16) per expert (an expert has at most T

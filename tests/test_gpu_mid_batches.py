@@ -2,7 +2,8 @@
 restatement of moe_ffn_batch (model.rs:286-371): three and four tokens (routed by a launch of their
 own), 8 to 15 tokens on the decode-batch kernels by default, Q6_K down on them, groups of 16 to 191
 members on average with Q6_K gate/up and down (k_gemm_r), and Q4_K groups whose member tiles of 64
-hold 1 to 4 tiles of 16 (k_gemm's sweeps), skewed groups among them.
+hold 1 to 4 tiles of 16 (k_gemm's sweeps), skewed groups among them; above 16 tokens, groups averaging
+fewer than 16 members on k_gemm_mid: one or two member tiles, further tiles of an expert, one member.
 """
 import numpy as np
 import pytest
@@ -50,3 +51,24 @@ def test_skewed_groups(ctx, oracle, gate, down):
     w = synth.moe_weights(5, hidden=512, moe_ff=512, n_experts=6, n_used=2, gate_dtype=gate, down_dtype=down, bias=bias)
     x = synth.hidden_states(9, 96, hidden=512)
     check_moe(ctx, oracle, w, x, 96, f"skewed groups {gate} {down}")
+
+
+# k_gemm_mid needs 160 blocks of 256 outputs: (hidden, moe_ff, experts, k, tokens, bias of expert 0)
+MID = [
+    (2048, 1792, 32, 4, 17, 0.0), (2048, 1280, 32, 4, 127, 0.0), (2048, 1536, 32, 2, 255, 0.0),
+    (1280, 1280, 32, 3, 33, 3.0), (1280, 1280, 32, 1, 161, 3.0),   # expert 0 chosen by every token
+    (1792, 2048, 23, 2, 65, 3.0), (512, 2048, 20, 2, 150, 0.0),    # down of 512 outputs: k_gemm
+]
+
+
+@pytest.mark.parametrize("case", MID, ids=lambda c: "-".join(map(str, c)))
+@pytest.mark.parametrize("down", [Q4_K, Q6_K])
+def test_groups_of_a_few(ctx, oracle, case, down):
+    hidden, ff, E, K, T, b0 = case
+    bias = np.zeros(E, np.float32)
+    bias[0] = b0
+    w = synth.moe_weights(T, hidden=hidden, moe_ff=ff, n_experts=E, n_used=K, gate_dtype=Q4_K, down_dtype=down,
+                          bias=bias)
+    x = synth.hidden_states(T + 1, T, hidden=hidden)
+    x[T // 2, :256] = 0.0
+    check_moe(ctx, oracle, w, x, T, f"groups of a few {case} {down}")
