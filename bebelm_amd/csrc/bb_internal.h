@@ -333,9 +333,9 @@ hipError_t launch_conv(hipStream_t s, bool op, const float* src, const float* st
                        int T, float* out);
 // state <- the last L-1 columns of [state; bx] (run after launch_conv on the same batch).
 hipError_t launch_conv_state(hipStream_t s, bool op, const float* src, float* state, int C, int L, int T);
-// One token: conv, state update and the Q8 of y in one launch (C % 256 == 0; y f32[C] too).
-hipError_t launch_conv1_q8(hipStream_t s, const float* src, float* state, const float* w, int C, int L, float* y,
-                           Q8Bufs q);
+// An op's conv, state update and the Q8 of its output in one launch (C % 256 == 0, 2 <= L <= CONV_Q8_L_MAX).
+constexpr int CONV_Q8_L_MAX = 16;
+hipError_t launch_conv_q8(hipStream_t s, const float* src, float* state, const float* w, int C, int L, int T, Q8Bufs q);
 // per-head rmsnorm (gain null: none) and RoPE from (cos, sin) rows [T][hd/2], in place on buf [T][n_heads][hd].
 hipError_t launch_norm_rope(hipStream_t s, float* buf, int T, int n_heads, int hd, const float* gain, float eps,
                             const float2* rope, float* buf2 = nullptr, int n2 = 0,

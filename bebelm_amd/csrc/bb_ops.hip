@@ -20,6 +20,7 @@
 //             cosf of the reference's angle sequence (theta from (float)pos, times
 //             powf(base, -2/d) per pair): the same functions the reference's f32 sin_cos calls.
 #include "bb_device.h"
+#include <algorithm>
 #include <utility>
 #include "bb_internal.h"
 
@@ -85,32 +86,47 @@ hipError_t launch_conv_state(hipStream_t s, bool op, const float* src, float* st
   return hipGetLastError();
 }
 
-// One token, the whole conv step in one launch: wave w takes channels 256w..256w+255 (four per
-// lane, lane l holding 4l..4l+3): y = C·conv over [state; bx] as k_conv computes it, the state
-// shifted by one column as k_conv_state does (each channel's reads before its writes, in the
-// same thread), and the 256-block of y quantised to Q8 (quantize_q8's arithmetic) for out_proj.
-__global__ void __launch_bounds__(64) k_conv1_q8(const float* __restrict__ src, float* state,
-                                                 const float* __restrict__ w, int C, int L, float* __restrict__ y,
-                                                 Q8Bufs q) {
-  const int c0 = blockIdx.x * QK + 4 * threadIdx.x;
-  float out[4];
+// The whole conv step of an op whose output is projected from Q8, in one launch: wave w of a block takes
+// token t = CONV_TOK·y + w of channels 256x..256x+255 (four per lane, lane l holding 4l..4l+3): C·conv
+// over [state; bx] as k_conv computes it, quantised (quantize_q8's arithmetic). A block of the first
+// row (y = 0) holds every token that reads the state, max(CONV_TOK, L - 1) of them, and its first wave
+// shifts the state as k_conv_state does once they have read it. Bound by its launch and one round of
+// loads: a 77-token op of hidden 2048 took 28.7 us with conv, state and Q8 as three launches, 24.1 with
+// this one.
+constexpr int CONV_TOK = 4;
+
+__global__ void __launch_bounds__(64 * CONV_Q8_L_MAX) k_conv_q8(const float* __restrict__ src, float* state,
+                                                                const float* __restrict__ w, int C, int L, int T,
+                                                                Q8Bufs q) {
+  const int lane = threadIdx.x & 63, c0 = blockIdx.x * QK + 4 * lane, tb = (int)(blockDim.x >> 6);
+  const int t = blockIdx.y * tb + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (t < T) {
+    float out[4];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int c = c0 + u;
-    const float* wc = w + (size_t)c * L;
-    float sum = wc[L - 1] * conv_col<true>(src, state, C, L, L - 1, c);
-    for (int k = 0; k + 1 < L; ++k) sum += wc[k] * conv_col<true>(src, state, C, L, k, c);
-    out[u] = src[C + c] * sum;
-    for (int k = 0; k + 1 < L; ++k) state[(size_t)k * C + c] = conv_col<true>(src, state, C, L, 1 + k, c);
+    for (int u = 0; u < 4; ++u) {
+      const int c = c0 + u;
+      const float* wc = w + (size_t)c * L;
+      float sum = wc[L - 1] * conv_col<true>(src, state, C, L, t + L - 1, c);
+      for (int k = 0; k + 1 < L; ++k) sum += wc[k] * conv_col<true>(src, state, C, L, t + k, c);
+      out[u] = src[(size_t)t * 3 * C + C + c] * sum;
+    }
+    wave_quantize_block(make_float4(out[0], out[1], out[2], out[3]), t, blockIdx.x, gridDim.x, q.q, q.scales, q.sums,
+                        q.tiled);
   }
-  *reinterpret_cast<float4*>(y + c0) = make_float4(out[0], out[1], out[2], out[3]);
-  wave_quantize_block(make_float4(out[0], out[1], out[2], out[3]), 0, blockIdx.x, gridDim.x, q.q, q.scales, q.sums, 0);
+  if (blockIdx.y > 0) return;  // the whole block
+  __syncthreads();             // the block's tokens have read the state
+  if (threadIdx.x < 64) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      for (int k = 0; k + 1 < L; ++k) state[(size_t)k * C + c0 + u] = conv_col<true>(src, state, C, L, T + k, c0 + u);
+  }
 }
 
-hipError_t launch_conv1_q8(hipStream_t s, const float* src, float* state, const float* w, int C, int L, float* y,
-                           Q8Bufs q) {
-  if (C % QK != 0 || L < 2 || !q.q) return hipErrorInvalidValue;
-  BB_LAUNCH(k_conv1_q8, dim3((unsigned)(C / QK)), dim3(64), 0, s, src, state, w, C, L, y, q);
+hipError_t launch_conv_q8(hipStream_t s, const float* src, float* state, const float* w, int C, int L, int T, Q8Bufs q) {
+  if (C % QK != 0 || L < 2 || L > CONV_Q8_L_MAX || T < 1 || !q.q) return hipErrorInvalidValue;
+  const int tb = std::min(std::max(CONV_TOK, L - 1), T);
+  BB_LAUNCH(k_conv_q8, dim3((unsigned)(C / QK), (unsigned)((T + tb - 1) / tb)), dim3(64 * tb), 0, s, src, state, w, C, L,
+            T, q);
   return hipGetLastError();
 }
 

@@ -16,7 +16,7 @@
 // model's matrices) time alike within 5%, one row or four 10% worse.
 // Arithmetic and order are those of the kernels named: k_residual_norm's f64 sum (thread j's
 // elements j, j + 256, ..., a butterfly, the four waves in a tree), k_rows_q8w's row values and
-// left-to-right sum from -0.0 (one token: matvec, matmul.rs:850), k_conv1_q8's conv.
+// left-to-right sum from -0.0 (one token: matvec, matmul.rs:850), k_conv_q8's conv.
 #include "bb_device.h"
 #include "bb_internal.h"
 

@@ -60,3 +60,18 @@ def test_attention_with_unpacked_projections(gpu_ctx, oracle):
         pos += t
     kv.close()
     op.close()
+
+
+@pytest.mark.parametrize("taps", [2, 3, 6, 16, 17])
+def test_conv_one_launch(gpu_ctx, oracle, taps):
+    # k_conv_q8: batches shorter and longer than the state, whole and partial groups of tokens (17 taps
+    # keep the separate kernels), each batch continuing from the state of the one before
+    w = synth.conv_weights(91 + taps, hidden=256, l_cache=taps, in_dtype=Q6_K, out_dtype=Q4_K)
+    op = ConvOp(gpu_ctx, w)
+    state = op.new_state()
+    for i, t in enumerate((2, 3, 1, 4, 5, 17, 8, 33)):
+        x = synth.hidden_states(50 + i, t, hidden=256).reshape(-1)
+        want, new = oracle.conv_forward(w, state, x, t)
+        assert_bits(op.forward(state, x, t, np.empty(t * 256, np.float32)), want, f"{taps} taps, {t} tokens")
+        assert_bits(state, new, f"{taps} taps, state after {t} tokens")
+    op.close()
