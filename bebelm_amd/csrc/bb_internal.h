@@ -214,8 +214,8 @@ hipError_t launch_gemm_gateup(hipStream_t s, int dtype, const uint8_t* gu, size_
                               float* aq_sx = nullptr, bool* quantized = nullptr, bool act_pad = false);
 hipError_t launch_gemm_down(hipStream_t s, int dtype, const uint8_t* dn, size_t stride_dn, int T, int H, int F, int E,
                             int K, const RouteBufs& rb, GemmX x, float* slots, bool act_pad = false);
-// Whether launch_gemm_down runs the down GEMM of this call as k_down16 (decode batches of Q4_K
-// experts, at most 16 members per expert).
+// Whether launch_gemm_down runs the down GEMM of this call as k_down16 (decode batches of at
+// most 16 tokens, so at most 16 members per expert).
 bool down16_applies(int dtype, int T, int H, int F, int E, int K);
 
 // A Q4_K / Q6_K weight matrix in the grouped GEMM's packed tile layout as a single expert: plain

@@ -2,17 +2,17 @@
 // short conv (model.rs:399-427 one token, :190-216 a batch) and GQA attention (model.rs:430-456,
 // :222-259), with their kernel-level pieces conv_step / conv_prefill (kernels/conv.rs:18-68),
 // softmax (kernels/softmax.rs:9-22), attention_decode (kernels/attention.rs:17-55) and the
-// per-head q/k norm + NEOX RoPE (model.rs:692-701, kernels/rope.rs:17-30). Projections run on
-// the Q4_K/Q6_K row kernels of bb_kernels.hip.
+// per-head q/k norm + NEOX RoPE (model.rs:692-701, kernels/rope.rs:17-30). The projections
+// are bb_row1.hip's (one token), bb_proj.hip's (batches) and bb_kernels.hip's.
 //
 // Exactness. Every value is computed with the reference's operations in its order:
 //   conv      sum = w[L-1]·bx, then += w[k]·col_k for k = 0..L-2 (columns oldest first; the
 //             columns before the batch come from the state). One thread per (token, channel):
 //             every output depends only on its own L columns, so the batch is the rolled loop.
-//   scores    matmul.rs's dot (32 fmaf chains, the `wide` lane reduce) in one lane per position,
-//             times 1/sqrt(head_dim).
-//   softmax   max, f32 exps (bb_expf: glibc's expf restated), their f64 sum left to right in one
-//             lane, each value times (float)(1.0 / sum).
+//   scores    matmul.rs's dot (32 fmaf chains, the `wide` lane reduce) in one lane per position
+//             or, in batches, its chains on single-step f32 MFMA; times 1/sqrt(head_dim).
+//   softmax   max, f32 exps (bb_expf: glibc's expf restated), their f64 sum left to right or
+//             a tree sum whose error bound settles (float)(1.0 / sum); each value times (float)(1.0 / sum).
 //   P·V       out[d] = Σ_j w_j·v[j][d] in position order from 0.0, one lane per d.
 //   q/k norm  rmsnorm over head_dim with its f64 sum left to right in one lane (the reference's
 //             order; the hidden-size rmsnorm kernel sums as a tree), then RoPE with (cos, sin)

@@ -2,8 +2,10 @@
 //
 //   k_dispatch      counts, offsets and the stable grouping of (token, slot) entries by
 //                   expert — token-ascending, slot-ascending within an expert (model.rs:316-322)
-//   k_gemm_q4/q6    grouped expert GEMM on int8 MFMA: gate/up + SwiGLU (model.rs:325-334),
-//                   down (model.rs:335-341)
+//   k_gemm*         grouped expert GEMM on int8 MFMA: gate/up + SwiGLU (model.rs:325-334), down
+//                   (model.rs:335-341): k_gateup16 and k_down16 (up to 16 tokens), k_gemm_mid
+//                   (groups averaging under 16 members), k_gemm, k_gemm_r (Q6_K), k_gemm_wide
+//                   (Q6_K down, large groups)
 //   k_quant_rows    Q8 of the act rows (quantize_q8, kernels/matmul.rs:141-160)
 //
 // Exactness. Each output is matmul's row dot (kernels/matmul.rs:211-300 Q4_K, :648-760 Q6_K):
@@ -1847,7 +1849,7 @@ static hipError_t launch_mid(hipStream_t s, const uint8_t* w, size_t stride_e, i
 
 // Q6_K down GEMMs whose groups hold this many members on average take k_gemm_wide (blocks of up
 // to 256 members). For config 4 (4096 tokens, Zipf-skewed groups) it runs the Q6_K down GEMM in
-// 228 µs against k_gemm's 274; the Q4_K gate/up GEMM, whose 3-pass epilogue and operand build
+// 228 µs against 274 on k_gemm in tiles of 128 members; the Q4_K gate/up GEMM, whose 3-pass epilogue and operand build
 // are heavier, runs in 578 µs against k_gemm's 442 at its two waves per SIMD, so gate/up and Q4_K
 // rows stay on k_gemm.
 constexpr int WIDE_MIN_AVG = 192;
