@@ -1628,9 +1628,12 @@ int bb_stack_forward(bb_ctx* c, bb_stack* s, const float* x, size_t T, float* h_
       const float* h = static_cast<const float*>(d[0]);
       float* const out = static_cast<float*>(d[1]);
       const size_t nl = s->layers.size();
-      if (nl == 0) {
-        check_hip(hipMemcpyAsync(out, h, T * H * 4, hipMemcpyDeviceToDevice, c->stream), "h copy");
-        return;
+      // a single layer's boundary reads the input while it writes the output: where they overlap without
+      // being the same rows, the input is copied first (deeper stacks read it only before they write)
+      const uintptr_t xi = reinterpret_cast<uintptr_t>(h), xo = reinterpret_cast<uintptr_t>(out);
+      if (nl == 1 && xi != xo && (xi < xo ? xo - xi : xi - xo) < T * H * 4) {
+        check_hip(hipMemcpyAsync(s->h, h, T * H * 4, hipMemcpyDeviceToDevice, c->stream), "h copy");
+        h = s->h;
       }
       auto next_h = [&] { return h == s->h ? s->h2 : s->h; };
       // one token: a dense layer takes the boundary before it as its input (row1_ok)

@@ -76,3 +76,28 @@ def test_stack_orders(gpu_ctx, oracle):
         stack.close()
         for _, layer in layers:
             layer.close()
+
+
+@pytest.mark.parametrize("kind", ["dense", "moe"])
+@pytest.mark.parametrize("t,shift", [(1, 4), (5, 512), (5, -512), (3, 0)])
+def test_stack_of_one_layer_in_overlapping_rows(gpu_ctx, oracle, kind, t, shift):
+    # the output may lie over the input, at another place too (device pointers, shift floats apart)
+    import torch
+
+    h = 512
+    w = (synth.dense_weights(73, hidden=h, ff=768) if kind == "dense" else
+         synth.moe_weights(73, hidden=h, moe_ff=256, n_experts=8, n_used=2))
+    gain = np.ones(h, np.float32)
+    layer = (DenseLayer if kind == "dense" else MoeLayer)(gpu_ctx, w)
+    stack = FfnStack(gpu_ctx, [(gain, layer)])
+    x = synth.hidden_states(74, t, hidden=h).reshape(-1)
+    buf = torch.zeros(1024 + t * h, device="cuda")
+    at = 512
+    xv, ov = buf[at:at + t * h], buf[at + shift:at + shift + t * h]
+    xv.copy_(torch.from_numpy(x))
+    torch.cuda.synchronize()
+    stack.forward(xv, t, ov)
+    gpu_ctx.synchronize()
+    assert_bits(ov.cpu().numpy(), oracle.ffn_stack([(gain, w)], x, t), f"{kind} t={t} shift {shift}")
+    stack.close()
+    layer.close()
