@@ -100,6 +100,9 @@ uint8_t* scratch_of(int device) {
 }
 }  // namespace
 
+// The default of bb_ctx_set_batched_min_entries.
+constexpr size_t BATCHED_MIN_ENTRIES = 64;
+
 struct bb_ctx {
   int device = 0;
   hipStream_t own = nullptr;
@@ -117,9 +120,8 @@ struct bb_ctx {
   std::vector<hipEvent_t> event_pool;
   double kernel_ms[bb::K_COUNT] = {};
   int64_t launches[bb::K_COUNT] = {};
-  size_t batched_min_entries = 64;  // T*k from which MoE calls take the grouped-GEMM path
-  bool batched_default = true;      // (not set by the caller)
-  int n_cu = 256;                   // compute units of the device
+  size_t batched_min_entries = BATCHED_MIN_ENTRIES;  // T*k from which MoE calls take the grouped-GEMM path
+  int n_cu = 256;                                    // compute units of the device
 };
 
 struct bb_tensor {
@@ -342,15 +344,15 @@ bool moe_act_pad(const bb_moe* m, size_t T) {
          bb::down16_applies((int)m->dn_dtype, (int)T, (int)m->H, (int)m->F, (int)m->E, (int)m->K);
 }
 
-// Whether a call of T tokens takes the grouped-GEMM kernels. Unless the caller set the line, layers
-// whose batch both decode-batch kernels serve take them from 32 entries: config 2's layer, GEMV path
+// Whether a call of T tokens takes the grouped-GEMM kernels. At the default line, layers whose batch
+// both decode-batch kernels serve take them from 32 entries: config 2's layer, GEMV path
 // and here, 7 tokens 45 and 42 us, 8 tokens 46.8 and 42.9 (Q6_K down 52.8 and 52.4), 12 tokens 57.6
 // and 46.2 (65.5 and 54.7), 15 tokens 67.3 and 49.5; at 6 tokens Q6_K 47.9 and 51.1.
 constexpr size_t DECODE_BATCH_MIN_ENTRIES = 32;
 bool moe_batched(const bb_ctx* c, const bb_moe* m, size_t T) {
   const size_t n_ent = T * (size_t)m->K;
   return n_ent >= c->batched_min_entries ||
-         (c->batched_default && n_ent >= DECODE_BATCH_MIN_ENTRIES && moe_act_pad(m, T));
+         (c->batched_min_entries == BATCHED_MIN_ENTRIES && n_ent >= DECODE_BATCH_MIN_ENTRIES && moe_act_pad(m, T));
 }
 
 MoeWs carve_moe(bb_ctx* c, const bb_moe* m, size_t T, bool batched, const WsRegion* fixed = nullptr) {
@@ -1171,7 +1173,6 @@ int bb_ctx_set_batched_min_entries(bb_ctx* c, size_t min_entries) {
   return guard([&] {
     need_ctx(c);
     c->batched_min_entries = min_entries;
-    c->batched_default = false;
   });
 }
 

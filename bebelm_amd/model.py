@@ -77,7 +77,7 @@ class Context:
         check(lib().bb_ctx_reset_stats(self.handle))
 
     def set_batched_min_entries(self, n):
-        """MoE calls with T*k >= n take the grouped-GEMM (batched) kernels."""
+        """MoE calls with T*k >= n take the grouped-GEMM (batched) kernels (64: the default rule)."""
         check(lib().bb_ctx_set_batched_min_entries(self.handle, int(n)))
 
     def kernel_stats(self):

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from bebelm_amd import synth
-from bebelm_amd.model import Context
+from bebelm_amd.model import Context, MoeLayer
 
 from test_gpu_parity import Q4_K, Q6_K, check_moe
 
@@ -72,3 +72,24 @@ def test_groups_of_a_few(ctx, oracle, case, down):
     x = synth.hidden_states(T + 1, T, hidden=hidden)
     x[T // 2, :256] = 0.0
     check_moe(ctx, oracle, w, x, T, f"groups of a few {case} {down}")
+
+
+def test_the_default_line_can_be_set_back(ctx):
+    # a layer that the decode-batch kernels serve from 32 entries, and one entry less than that line
+    layer = MoeLayer(ctx, synth.moe_weights(3, hidden=512, moe_ff=1024, n_experts=32, n_used=4))
+
+    def kernels(t):
+        ctx.reset_stats()
+        ctx.profile(True)
+        layer.forward(synth.hidden_states(3, t, hidden=512).reshape(-1), t, np.empty(t * 512, np.float32))
+        ctx.synchronize()
+        ctx.profile(False)
+        return set(ctx.kernel_stats())
+
+    fresh = [kernels(t) for t in (7, 8)]
+    assert "gemm_gateup" not in fresh[0] and "gemm_gateup" in fresh[1]
+    ctx.set_batched_min_entries(1 << 40)
+    assert "gemm_gateup" not in kernels(8)
+    ctx.set_batched_min_entries(64)
+    assert [kernels(t) for t in (7, 8)] == fresh
+    layer.close()
