@@ -958,8 +958,7 @@ void conv_forward_dev(bb_ctx* c, bb_conv_op* op, float* state, const float* x, s
     if (gemm) rb = one_group(c, grp, T);
     const bb::RouteBufs* rbp = gemm ? &rb : nullptr;
     project_dev(c, op->in_proj, op->in_p, rbp, H, 3 * H, x, T, bcx, xq_in ? *xq_in : xq, xq_in != nullptr);
-    // (launch_conv_q8's grid has a row per four tokens or more)
-    if (quantised(op->out_proj) && op->L >= 2 && op->L <= bb::CONV_Q8_L_MAX && T <= 4 * size_t(65535)) {
+    if (quantised(op->out_proj) && bb::conv_q8_applies(op->L, T)) {
       // conv, state update and y's Q8 in one launch
       launch(c, bb::K_CONV, [&] { return bb::launch_conv_q8(c->stream, bcx, state, op->conv_w, (int)H, op->L, (int)T, yq); });
       project_dev(c, op->out_proj, op->out_p, rbp, H, H, y, T, out, yq, true);

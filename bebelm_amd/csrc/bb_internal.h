@@ -333,8 +333,10 @@ hipError_t launch_conv(hipStream_t s, bool op, const float* src, const float* st
                        int T, float* out);
 // state <- the last L-1 columns of [state; bx] (run after launch_conv on the same batch).
 hipError_t launch_conv_state(hipStream_t s, bool op, const float* src, float* state, int C, int L, int T);
-// An op's conv, state update and the Q8 of its output in one launch (C % 256 == 0, 2 <= L <= CONV_Q8_L_MAX).
+// An op's conv, state update and the Q8 of its output in one launch (C % 256 == 0), for filters of up to
+// CONV_Q8_L_MAX taps, or of any length for one token.
 constexpr int CONV_Q8_L_MAX = 16;
+bool conv_q8_applies(int L, size_t T);
 hipError_t launch_conv_q8(hipStream_t s, const float* src, float* state, const float* w, int C, int L, int T, Q8Bufs q);
 // per-head rmsnorm (gain null: none) and RoPE from (cos, sin) rows [T][hd/2], in place on buf [T][n_heads][hd].
 hipError_t launch_norm_rope(hipStream_t s, float* buf, int T, int n_heads, int hd, const float* gain, float eps,

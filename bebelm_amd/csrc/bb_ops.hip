@@ -86,47 +86,139 @@ hipError_t launch_conv_state(hipStream_t s, bool op, const float* src, float* st
   return hipGetLastError();
 }
 
-// The whole conv step of an op whose output is projected from Q8, in one launch: wave w of a block takes
-// token t = CONV_TOK·y + w of channels 256x..256x+255 (four per lane, lane l holding 4l..4l+3): C·conv
-// over [state; bx] as k_conv computes it, quantised (quantize_q8's arithmetic). A block of the first
-// row (y = 0) holds every token that reads the state, max(CONV_TOK, L - 1) of them, and its first wave
-// shifts the state as k_conv_state does once they have read it. Bound by its launch and one round of
-// loads: a 77-token op of hidden 2048 took 28.7 us with conv, state and Q8 as three launches, 24.1 with
-// this one.
-constexpr int CONV_TOK = 4;
+// The whole conv step of an op whose output is projected from Q8, in one launch: a wave takes TPW tokens
+// of channels 256x..256x+255 (four per lane, lane l holding 4l..4l+3): C·conv over [state; bx] as k_conv
+// computes it, quantised (quantize_q8's arithmetic). LM: taps of the filter, exactly (up to 4) or at
+// most. The first row of blocks (y = 0) holds every token that reads the state (4·TPW >= LM - 1), and
+// its first wave shifts the state as k_conv_state does once they have read it.
+// Bound by a launch and one round of loads up to a few hundred tokens, then by the rows' bytes: every
+// tap, column and C value is loaded before the first product, so a wave waits for memory once. (A form
+// whose lanes walked the taps of one channel after the other waited a dozen times: hidden 2048, 3
+// taps, it and this one 12.0 and 4.3 us at 512 tokens, 71.7 and 15.9 at 4096; hidden 1024, 16 taps,
+// 58.5 and 14.4 at 512. k_conv, k_conv_state and the Q8 as three launches: 13.8, 44.2 and 26.6.)
+// Up to 4 taps a token a wave is best (4096 tokens of hidden 2048: 18.3 us with four); longer filters
+// share the columns of four tokens, which also lets a block hold the tokens that read the state.
+constexpr int CONV_WAVES = 4;
 
-__global__ void __launch_bounds__(64 * CONV_Q8_L_MAX) k_conv_q8(const float* __restrict__ src, float* state,
-                                                                const float* __restrict__ w, int C, int L, int T,
-                                                                Q8Bufs q) {
-  const int lane = threadIdx.x & 63, c0 = blockIdx.x * QK + 4 * lane, tb = (int)(blockDim.x >> 6);
-  const int t = blockIdx.y * tb + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (t < T) {
-    float out[4];
+// Columns t (four channels from c0) of [state; bx], t < 0 in the state, t >= T the last one again.
+struct ConvCol {
+  float4 b, x;
+  bool old;
+  __device__ __forceinline__ void load(const float* __restrict__ src, const float* state, int C, int L, int T, int t,
+                                       int c0) {
+    t = min(t, T - 1);
+    old = t < 0;
+    const float* p = old ? state + (size_t)max(t + L - 1, 0) * C : src + (size_t)t * 3 * C;
+    b = *reinterpret_cast<const float4*>(p + c0);
+    x = *reinterpret_cast<const float4*>((old ? p : p + 2 * C) + c0);
+  }
+  __device__ __forceinline__ float4 value() const {
+    return old ? b : make_float4(b.x * x.x, b.y * x.y, b.z * x.z, b.w * x.w);
+  }
+};
+
+template <int LM, int TPW>
+__global__ void __launch_bounds__(64 * CONV_WAVES) k_conv_q8(const float* __restrict__ src, float* state,
+                                                             const float* __restrict__ w, int C, int Lr, int T,
+                                                             Q8Bufs q) {
+  static_assert(CONV_WAVES * TPW >= LM - 1, "the first blocks hold every token that reads the state");
+  constexpr int NC = LM - 1 + TPW;
+  const int L = LM <= 4 ? LM : Lr;
+  const int lane = threadIdx.x & 63, c0 = blockIdx.x * QK + 4 * lane;
+  const int t0 = (blockIdx.y * CONV_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * TPW;
+  if (t0 < T) {
+    // tap[u][k]: channel c0 + u, the tap of the column k - (LM - 1) tokens on
+    float tap[4][LM];
+    const float* wc = w + (size_t)c0 * L;
+    if constexpr (LM <= 4) {
+      float4 v[LM];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int c = c0 + u;
-      const float* wc = w + (size_t)c * L;
-      float sum = wc[L - 1] * conv_col<true>(src, state, C, L, t + L - 1, c);
-      for (int k = 0; k + 1 < L; ++k) sum += wc[k] * conv_col<true>(src, state, C, L, t + k, c);
-      out[u] = src[(size_t)t * 3 * C + C + c] * sum;
+      for (int i = 0; i < LM; ++i) v[i] = reinterpret_cast<const float4*>(wc)[i];
+#pragma unroll
+      for (int i = 0; i < 4 * LM; ++i) tap[i / LM][i % LM] = reinterpret_cast<const float*>(v)[i];
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int k = 0; k < LM; ++k) tap[u][k] = wc[u * L + max(k - (LM - L), 0)];
     }
-    wave_quantize_block(make_float4(out[0], out[1], out[2], out[3]), t, blockIdx.x, gridDim.x, q.q, q.scales, q.sums,
-                        q.tiled);
+    ConvCol col[NC];
+#pragma unroll
+    for (int j = 0; j < NC; ++j) col[j].load(src, state, C, L, T, t0 + j - (LM - 1), c0);
+    float4 cc[TPW];
+#pragma unroll
+    for (int i = 0; i < TPW; ++i)
+      cc[i] = *reinterpret_cast<const float4*>(src + (size_t)min(t0 + i, T - 1) * 3 * C + C + c0);
+    __builtin_amdgcn_sched_barrier(0);
+    float4 bx[NC];
+#pragma unroll
+    for (int j = 0; j < NC; ++j) bx[j] = col[j].value();
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) {
+      if (t0 + i >= T) break;
+      float out[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        float sum = tap[u][LM - 1] * reinterpret_cast<const float*>(&bx[i + LM - 1])[u];
+#pragma unroll
+        for (int k = 0; k + 1 < LM; ++k)
+          if (LM <= 4 || k >= LM - L) sum += tap[u][k] * reinterpret_cast<const float*>(&bx[i + k])[u];
+        out[u] = reinterpret_cast<const float*>(&cc[i])[u] * sum;
+      }
+      wave_quantize_block(make_float4(out[0], out[1], out[2], out[3]), t0 + i, blockIdx.x, gridDim.x, q.q, q.scales,
+                          q.sums, q.tiled);
+    }
   }
   if (blockIdx.y > 0) return;  // the whole block
   __syncthreads();             // the block's tokens have read the state
   if (threadIdx.x < 64) {
+    ConvCol col[LM - 1];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-      for (int k = 0; k + 1 < L; ++k) state[(size_t)k * C + c0 + u] = conv_col<true>(src, state, C, L, T + k, c0 + u);
+    for (int k = 0; k + 1 < LM; ++k) col[k].load(src, state, C, L, T, T - (L - 1) + min(k, L - 2), c0);
+#pragma unroll
+    for (int k = 0; k + 1 < LM; ++k)
+      if (k + 1 < L) *reinterpret_cast<float4*>(state + (size_t)k * C + c0) = col[k].value();
   }
 }
 
+// One token and a filter of any length.
+__global__ void __launch_bounds__(64) k_conv1_q8(const float* __restrict__ src, float* state,
+                                                 const float* __restrict__ w, int C, int L, Q8Bufs q) {
+  const int c0 = blockIdx.x * QK + 4 * threadIdx.x;
+  float out[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int c = c0 + u;
+    const float* wc = w + (size_t)c * L;
+    float sum = wc[L - 1] * conv_col<true>(src, state, C, L, L - 1, c);
+    for (int k = 0; k + 1 < L; ++k) sum += wc[k] * conv_col<true>(src, state, C, L, k, c);
+    out[u] = src[C + c] * sum;
+    for (int k = 0; k + 1 < L; ++k) state[(size_t)k * C + c] = conv_col<true>(src, state, C, L, 1 + k, c);
+  }
+  wave_quantize_block(make_float4(out[0], out[1], out[2], out[3]), 0, blockIdx.x, gridDim.x, q.q, q.scales, q.sums,
+                      q.tiled);
+}
+
+bool conv_q8_applies(int L, size_t T) {
+  return L >= 2 && (T == 1 || (L <= CONV_Q8_L_MAX && T <= (size_t)CONV_WAVES * 65535));  // (a row of blocks per 4 tokens or more)
+}
+
 hipError_t launch_conv_q8(hipStream_t s, const float* src, float* state, const float* w, int C, int L, int T, Q8Bufs q) {
-  if (C % QK != 0 || L < 2 || L > CONV_Q8_L_MAX || T < 1 || !q.q) return hipErrorInvalidValue;
-  const int tb = std::min(std::max(CONV_TOK, L - 1), T);
-  BB_LAUNCH(k_conv_q8, dim3((unsigned)(C / QK), (unsigned)((T + tb - 1) / tb)), dim3(64 * tb), 0, s, src, state, w, C, L,
-            T, q);
+  if (C % QK != 0 || T < 1 || !conv_q8_applies(L, T) || !q.q) return hipErrorInvalidValue;
+  const unsigned cb = (unsigned)(C / QK);
+  if (L > CONV_Q8_L_MAX) {
+    BB_LAUNCH(k_conv1_q8, dim3(cb), dim3(64), 0, s, src, state, w, C, L, q);
+    return hipGetLastError();
+  }
+#define BB_CONV_Q8(lm, tpw)                                                                                            \
+  BB_LAUNCH((k_conv_q8<lm, tpw>), dim3(cb, (unsigned)((T + CONV_WAVES * tpw - 1) / (CONV_WAVES * tpw))),               \
+            dim3(64 * CONV_WAVES), 0, s, src, state, w, C, L, T, q)
+  if (L == 2) BB_CONV_Q8(2, 1);
+  else if (L == 3) BB_CONV_Q8(3, 1);
+  else if (L == 4) BB_CONV_Q8(4, 1);
+  else if (L <= 8) BB_CONV_Q8(8, 4);
+  else BB_CONV_Q8(16, 4);
+#undef BB_CONV_Q8
   return hipGetLastError();
 }
 
