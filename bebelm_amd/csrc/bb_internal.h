@@ -334,7 +334,8 @@ hipError_t launch_conv(hipStream_t s, bool op, const float* src, const float* st
 // state <- the last L-1 columns of [state; bx] (run after launch_conv on the same batch).
 hipError_t launch_conv_state(hipStream_t s, bool op, const float* src, float* state, int C, int L, int T);
 // An op's conv, state update and the Q8 of its output in one launch (C % 256 == 0), for filters of up to
-// CONV_Q8_L_MAX taps, or of any length for one token.
+// CONV_Q8_L_MAX taps (longer ones keep the three kernels: one token and 20 taps 13 us with them, 24 in
+// one launch of four wavefronts whose lanes walk the taps).
 constexpr int CONV_Q8_L_MAX = 16;
 bool conv_q8_applies(int L, size_t T);
 hipError_t launch_conv_q8(hipStream_t s, const float* src, float* state, const float* w, int C, int L, int T, Q8Bufs q);

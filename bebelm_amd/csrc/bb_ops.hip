@@ -181,35 +181,13 @@ __global__ void __launch_bounds__(64 * CONV_WAVES) k_conv_q8(const float* __rest
   }
 }
 
-// One token and a filter of any length.
-__global__ void __launch_bounds__(64) k_conv1_q8(const float* __restrict__ src, float* state,
-                                                 const float* __restrict__ w, int C, int L, Q8Bufs q) {
-  const int c0 = blockIdx.x * QK + 4 * threadIdx.x;
-  float out[4];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int c = c0 + u;
-    const float* wc = w + (size_t)c * L;
-    float sum = wc[L - 1] * conv_col<true>(src, state, C, L, L - 1, c);
-    for (int k = 0; k + 1 < L; ++k) sum += wc[k] * conv_col<true>(src, state, C, L, k, c);
-    out[u] = src[C + c] * sum;
-    for (int k = 0; k + 1 < L; ++k) state[(size_t)k * C + c] = conv_col<true>(src, state, C, L, 1 + k, c);
-  }
-  wave_quantize_block(make_float4(out[0], out[1], out[2], out[3]), 0, blockIdx.x, gridDim.x, q.q, q.scales, q.sums,
-                      q.tiled);
-}
-
 bool conv_q8_applies(int L, size_t T) {
-  return L >= 2 && (T == 1 || (L <= CONV_Q8_L_MAX && T <= (size_t)CONV_WAVES * 65535));  // (a row of blocks per 4 tokens or more)
+  return L >= 2 && L <= CONV_Q8_L_MAX && T <= (size_t)CONV_WAVES * 65535;  // (a row of blocks per 4 tokens or more)
 }
 
 hipError_t launch_conv_q8(hipStream_t s, const float* src, float* state, const float* w, int C, int L, int T, Q8Bufs q) {
   if (C % QK != 0 || T < 1 || !conv_q8_applies(L, T) || !q.q) return hipErrorInvalidValue;
   const unsigned cb = (unsigned)(C / QK);
-  if (L > CONV_Q8_L_MAX) {
-    BB_LAUNCH(k_conv1_q8, dim3(cb), dim3(64), 0, s, src, state, w, C, L, q);
-    return hipGetLastError();
-  }
 #define BB_CONV_Q8(lm, tpw)                                                                                            \
   BB_LAUNCH((k_conv_q8<lm, tpw>), dim3(cb, (unsigned)((T + CONV_WAVES * tpw - 1) / (CONV_WAVES * tpw))),               \
             dim3(64 * CONV_WAVES), 0, s, src, state, w, C, L, T, q)

@@ -89,21 +89,3 @@ def test_conv_in_groups_of_tokens(gpu_ctx, oracle, taps):
         assert_bits(op.forward(state, x, t, np.empty(t * 512, np.float32)), want, f"{taps} taps, {t} tokens")
         assert_bits(state, new, f"{taps} taps, state after {t} tokens")
     op.close()
-
-
-def test_one_token_of_a_long_filter_is_one_conv_launch(gpu_ctx, oracle):
-    w = synth.conv_weights(130, hidden=256, l_cache=20)
-    op = ConvOp(gpu_ctx, w)
-    state = op.new_state()
-    state[:] = synth.hidden_states(131, 19, hidden=256).reshape(-1)
-    gpu_ctx.reset_stats()
-    gpu_ctx.profile(True)
-    for i in range(2):
-        x = synth.hidden_states(132 + i, 1, hidden=256).reshape(-1)
-        want, new = oracle.conv_forward(w, state, x, 1)
-        assert_bits(op.forward(state, x, 1, np.empty(256, np.float32)), want, f"token {i}")
-        assert_bits(state, new, f"state after token {i}")
-    gpu_ctx.profile(False)
-    stats = gpu_ctx.kernel_stats()
-    assert "conv_state" not in stats and stats["conv"][1] == 2, stats
-    op.close()
