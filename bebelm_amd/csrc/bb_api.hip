@@ -335,24 +335,40 @@ struct WsRegion {
   size_t cap = 0;
 };
 
-// Decode batches whose gate/up and down GEMMs both run as the kernels of at most 16 members
-// (k_gateup16, k_down16): the Q8 act rows of expert e's member m go to row 16e + m (E·16 rows).
-bool moe_act_pad(const bb_moe* m, size_t T) {
-  const int n_ent = (int)(T * m->K);
+// Whether the gate/up GEMM of T tokens runs as k_gateup16 (decode batches of at most 16 tokens).
+bool moe_gateup16(const bb_moe* m, size_t T) {
   return bb::gateup16_applies((int)m->gu_dtype, (int)T, (int)m->H, (int)m->F, (int)m->E, (int)m->K,
-                              !bb::gemm_reads_ms((int)m->dn_dtype, n_ent, (int)m->E)) &&
+                              !bb::gemm_reads_ms((int)m->dn_dtype, (int)(T * m->K), (int)m->E));
+}
+
+// Decode batches whose down GEMM runs as k_down16 too: the Q8 act rows of expert e's member m go to row
+// 16e + m (E·16 rows).
+bool moe_act_pad(const bb_moe* m, size_t T) {
+  return moe_gateup16(m, T) &&
          bb::down16_applies((int)m->dn_dtype, (int)T, (int)m->H, (int)m->F, (int)m->E, (int)m->K);
 }
 
-// Whether a call of T tokens takes the grouped-GEMM kernels. At the default line, layers whose batch
-// both decode-batch kernels serve take them from 32 entries: config 2's layer, GEMV path
-// and here, 7 tokens 45 and 42 us, 8 tokens 46.8 and 42.9 (Q6_K down 52.8 and 52.4), 12 tokens 57.6
-// and 46.2 (65.5 and 54.7), 15 tokens 67.3 and 49.5; at 6 tokens Q6_K 47.9 and 51.1.
-constexpr size_t DECODE_BATCH_MIN_ENTRIES = 32;
+// The entries from which a layer whose gate/up k_gateup16 serves takes the batched kernels at the default
+// line. Their time hardly depends on the entries (config 2's layer 40.7 us at 8 tokens, 43.4 at 15),
+// the GEMV path's grows with them (50.8 and 62.7) and with the expert rows, but it needs no launch for
+// the route and cuts a layer of few blocks finer. So the line follows the gate/up blocks (E·ff/256).
+// Hidden 2048, Q4_K down, GEMV path and batched: 8 experts of 512 (16 blocks) 25 and 35 us at 32
+// entries, 31 and 36 at 60; 16 of 1024 (64) 34 and 37, 40 and 38; 20 of 1024 (80) 37 and 37, at 40
+// entries 46 and 38; 12 of 1792 (84) 44 and 41; 32 of 1024 (128) 38 and 37. Hidden 512, where the
+// routes are cheap: 8 experts of 1024 (32) 25 and 26 at 32 entries, 29 and 26 at 40, 32 experts 26 and
+// 25; with Q6_K down (k_gemm there) 28 and 30 at 32, 30 and 30 at 48 (8 tokens and k = 8: 32 and 31).
+size_t decode_batch_min_entries(const bb_moe* m) {
+  const size_t blocks = (size_t)m->E * m->F / 256;
+  if (m->H > 1024) return blocks < 80 ? BATCHED_MIN_ENTRIES : std::max<size_t>(32, (2688 + blocks - 1) / blocks);
+  if (m->dn_dtype == BB_Q6_K) return 48;
+  return blocks < 48 ? 40 : 32;
+}
+
+// Whether a call of T tokens takes the grouped-GEMM kernels.
 bool moe_batched(const bb_ctx* c, const bb_moe* m, size_t T) {
   const size_t n_ent = T * (size_t)m->K;
-  return n_ent >= c->batched_min_entries ||
-         (c->batched_min_entries == BATCHED_MIN_ENTRIES && n_ent >= DECODE_BATCH_MIN_ENTRIES && moe_act_pad(m, T));
+  return n_ent >= c->batched_min_entries || (c->batched_min_entries == BATCHED_MIN_ENTRIES &&
+                                             n_ent >= decode_batch_min_entries(m) && moe_gateup16(m, T));
 }
 
 MoeWs carve_moe(bb_ctx* c, const bb_moe* m, size_t T, bool batched, const WsRegion* fixed = nullptr) {

@@ -1253,9 +1253,13 @@ bool gateup16_applies(int dtype, int T, int H, int F, int E, int K, bool act_q8)
          F % QK == 0 && (H == 2048 || H == 512);
 }
 
+// Q6_K rows on fewer blocks (E·H/256) than this stay on k_gemm, whose blocks of 128 rows leave fewer CUs
+// idle: 64 entries, a layer with k_gemm and with k_down16: 64 blocks 48 and 51 us, 128 blocks 49
+// and 50, 160 blocks 57 and 50, 256 blocks 58 and 53 (hidden 2048, ff 1792); 64 blocks of 512 37.2 and 37.6.
+constexpr int DN16_Q6_MIN_BLOCKS = 160;
 bool down16_applies(int dtype, int T, int H, int F, int E, int K) {
   const int n_ent = T * K;
-  return (dtype == DT_Q4_K || dtype == DT_Q6_K) && gemm_member_tiles(n_ent, E) == 1 && T <= 16 && n_ent <= 64 &&
+  return (dtype == DT_Q4_K || (dtype == DT_Q6_K && E * (H / 256) >= DN16_Q6_MIN_BLOCKS)) && gemm_member_tiles(n_ent, E) == 1 && T <= 16 && n_ent <= 64 &&
          H % 256 == 0 && F % QK == 0 && F / QK >= 1 && F / QK <= 8;
 }
 

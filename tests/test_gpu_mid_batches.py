@@ -74,22 +74,55 @@ def test_groups_of_a_few(ctx, oracle, case, down):
     check_moe(ctx, oracle, w, x, T, f"groups of a few {case} {down}")
 
 
+def kernels(ctx, layer, hidden, t):
+    """The kernels that a call of t tokens launches."""
+    ctx.reset_stats()
+    ctx.profile(True)
+    layer.forward(synth.hidden_states(3, t, hidden=hidden).reshape(-1), t, np.empty(t * hidden, np.float32))
+    ctx.synchronize()
+    ctx.profile(False)
+    return set(ctx.kernel_stats())
+
+
 def test_the_default_line_can_be_set_back(ctx):
     # a layer that the decode-batch kernels serve from 32 entries, and one entry less than that line
     layer = MoeLayer(ctx, synth.moe_weights(3, hidden=512, moe_ff=1024, n_experts=32, n_used=4))
-
-    def kernels(t):
-        ctx.reset_stats()
-        ctx.profile(True)
-        layer.forward(synth.hidden_states(3, t, hidden=512).reshape(-1), t, np.empty(t * 512, np.float32))
-        ctx.synchronize()
-        ctx.profile(False)
-        return set(ctx.kernel_stats())
-
-    fresh = [kernels(t) for t in (7, 8)]
+    fresh = [kernels(ctx, layer, 512, t) for t in (7, 8)]
     assert "gemm_gateup" not in fresh[0] and "gemm_gateup" in fresh[1]
     ctx.set_batched_min_entries(1 << 40)
-    assert "gemm_gateup" not in kernels(8)
+    assert "gemm_gateup" not in kernels(ctx, layer, 512, 8)
     ctx.set_batched_min_entries(64)
-    assert [kernels(t) for t in (7, 8)] == fresh
+    assert [kernels(ctx, layer, 512, t) for t in (7, 8)] == fresh
     layer.close()
+
+
+# (hidden, moe_ff, experts, k, down, tokens on the GEMV path, tokens on the batched one)
+LINES = [
+    (2048, 512, 8, 4, Q4_K, 15, 16), (2048, 1024, 4, 2, Q6_K, 16, 32), (2048, 1024, 16, 8, Q4_K, 7, 8),
+    (2048, 1024, 20, 4, Q4_K, 8, 9), (2048, 1792, 12, 2, Q4_K, 15, 16), (512, 1024, 8, 8, Q4_K, 4, 5),
+    (512, 1024, 12, 4, Q4_K, 7, 8), (512, 1024, 12, 4, Q6_K, 11, 12), (1024, 1024, 16, 4, Q4_K, 15, 16),
+]
+
+
+@pytest.mark.parametrize("case", LINES, ids=lambda c: "-".join(map(str, c)))
+def test_the_default_line(ctx, case):
+    # layers of few gate/up blocks keep the GEMV path longer
+    hidden, ff, E, K, down, t0, t1 = case
+    layer = MoeLayer(ctx, synth.moe_weights(4, hidden=hidden, moe_ff=ff, n_experts=E, n_used=K, gate_dtype=Q4_K,
+                                            down_dtype=down))
+    assert "gemm_gateup" not in kernels(ctx, layer, hidden, t0)
+    assert "gemm_gateup" in kernels(ctx, layer, hidden, t1)
+    layer.close()
+
+
+# Q6_K down on k_down16: 160 blocks of 256 rows and more; rows of 1 to 8 super-blocks, and one case below
+@pytest.mark.parametrize("case", [(2048, 256, 20, 4, 16), (2048, 512, 23, 3, 9), (1280, 1280, 32, 4, 16),
+                                  (1792, 2048, 23, 5, 12), (2048, 768, 19, 4, 16)],
+                         ids=lambda c: "-".join(map(str, c)))
+def test_q6_down_of_decode_batches(ctx, oracle, case):
+    hidden, ff, E, K, T = case
+    w = synth.moe_weights(T, hidden=hidden, moe_ff=ff, n_experts=E, n_used=K, gate_dtype=Q4_K, down_dtype=Q6_K)
+    x = synth.hidden_states(T + 2, T, hidden=hidden)
+    ctx.set_batched_min_entries(1)
+    check_moe(ctx, oracle, w, x, T, f"decode batch {case}")
+    ctx.set_batched_min_entries(64)
