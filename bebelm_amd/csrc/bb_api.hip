@@ -465,11 +465,14 @@ MoeWs moe_forward_dev(bb_ctx* c, bb_moe* m, const float* x, size_t T, float* out
     const int batch_mode = T > 1;
     const int max_hit = (int)std::min<size_t>((size_t)m->E, n_ent);
     // one or two tokens: every gate/up block routes them itself (or, up to four, only gates them, from
-    // logits computed before the call). With three the blocks' own routes already cost more than a
-    // launch (config 2's layer: 3 tokens 38 us against 34, 4 tokens 44 against 37).
+    // logits computed before the call). With three the blocks' own routes, whose time follows the rows
+    // they read (T x hidden), cost more than a launch, unless the rows are short: layer with the blocks'
+    // routes and with a launch, hidden 2048 3 tokens 36 and 32 us, 4 tokens 42 and 36 (32 experts; with 4
+    // 23 and 22, 24 and 22), hidden 1024 22 and 22, 26 and 24, hidden 512 18.2 and 20.0, 18.5 and 19.1
+    // (4 experts; with 20 21.0 and 21.4, 24.2 and 23.6).
     need(!pre || T <= (size_t)bb::ROUTE_IN_GATEUP_MAX_T, BB_ERR_ARG,
          "routes computed before the call serve at most 4 tokens");
-    const bool route_in = pre || T <= 2;
+    const bool route_in = pre || T <= 2 || (T <= (size_t)bb::ROUTE_IN_GATEUP_MAX_T && T * (size_t)m->H <= 2048);
     if (!route_in)
       launch(c, bb::K_ROUTE, [&] {
         return bb::launch_route(c->stream, m->router_cm, m->bias_dev, x, (int)T, m->H, m->E, m->K, 1, w.xq, w.rb);

@@ -126,3 +126,15 @@ def test_q6_down_of_decode_batches(ctx, oracle, case):
     ctx.set_batched_min_entries(1)
     check_moe(ctx, oracle, w, x, T, f"decode batch {case}")
     ctx.set_batched_min_entries(64)
+
+
+# (hidden, experts, k, tokens, a launch for the route): three and four tokens
+@pytest.mark.parametrize("case", [(512, 8, 2, 3, False), (512, 20, 2, 4, False), (768, 8, 2, 3, True), (1024, 8, 4, 4, True)],
+                         ids=lambda c: "-".join(map(str, c)))
+def test_routes_of_three_and_four_tokens(ctx, oracle, case):
+    hidden, E, K, T, launch = case
+    w = synth.moe_weights(T + E, hidden=hidden, moe_ff=512, n_experts=E, n_used=K)
+    layer = MoeLayer(ctx, w)
+    assert ("route_gating" in kernels(ctx, layer, hidden, T)) == launch
+    layer.close()
+    check_moe(ctx, oracle, w, synth.hidden_states(T + 3, T, hidden=hidden), T, f"routes {case}")
