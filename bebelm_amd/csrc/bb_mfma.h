@@ -113,50 +113,65 @@ __device__ __forceinline__ void q4_step_ops(const uint4 qv, int h, const Q4Lane&
   }
 }
 
+// The super-block against MT member tiles, the operands of a step fed to the tiles' MFMAs right away (few
+// live registers). built() runs once the operands no longer need the weight words.
+template <int MT, class Built>
+__device__ __forceinline__ void q4_steps(const uint4 hd, const uint4 (&qv)[2], const uint8_t* xb, const float* sb,
+                                         float (&acc)[MT][4], Built&& built) {
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const Q4Lane L = q4_lane(hd, g);
+  v4i D[MT][3];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int p = 0; p < 3; ++p) D[mt][p] = (v4i){0, 0, 0, 0};
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    v4i Bh, Bl;
+    q4_step_ops(qv[s & 1], s >> 1, L, Bh, Bl);
+    const int mv = L.ms[s >> 1];
+    const v4i Bm = {mv, mv, mv, mv};
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const v4i ax = read_x16(xb, mt * 16 + r, 4 * g + s);
+      D[mt][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ax, Bh, D[mt][0], 0, 0, 0);
+      D[mt][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ax, Bl, D[mt][1], 0, 0, 0);
+      D[mt][2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ax, Bm, D[mt][2], 0, 0, 0);
+    }
+  }
+  built();
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const float4 sx4 = *reinterpret_cast<const float4*>(sb + mt * 16 + 4 * g);
+    const float sxv[4] = {sx4.x, sx4.y, sx4.z, sx4.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int sd = 8 * D[mt][0][i] + D[mt][1][i];
+      const float v = sxv[i] * ((L.dd * (float)sd) - (L.dm * (float)D[mt][2][i]));
+      acc[mt][i] += v;
+    }
+  }
+}
+
 // MF: the min term sm from the members' sum records in msb (min_split_record: member m's 16
 // halves at msb + 32m, lane group g's four at + 8g) by one f16 MFMA per member tile, against
 // weights [64·m_{2g}, 64·m_{2g+1}, m_{2g}, m_{2g+1}]: sm arrives as an exact f32, instead of a
 // third int8 pass over the block (four MFMAs) and a conversion.
-// built() runs once the operands no longer need the weight words.
-template <int MT, bool MF = false, class Built>
+template <int MT, bool MF = false>
 __device__ __forceinline__ void q4_tiles(const uint4 hd, const uint4 (&qv)[2], const uint8_t* xb, const float* sb,
-                                         const uint8_t* msb, float (&acc)[MT][4], Built&& built) {
+                                         const uint8_t* msb, float (&acc)[MT][4]) {
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  if constexpr (MT == 1) return q4_steps<1>(hd, qv, xb, sb, acc, [] {});
   const Q4Lane L = q4_lane(hd, g);
   v4i Bm[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) Bm[h] = (v4i){L.ms[h], L.ms[h], L.ms[h], L.ms[h]};
-  if constexpr (MT == 1) {
-    // one member tile: the operands of step s feed its three MFMAs right away (fewer live
-    // registers, so more blocks fit on a CU)
-    v4i Dh = {0, 0, 0, 0}, Dl = {0, 0, 0, 0}, Dm = {0, 0, 0, 0};
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      v4i Bh, Bl;
-      q4_step_ops(qv[s & 1], s >> 1, L, Bh, Bl);
-      const v4i ax = read_x16(xb, r, 4 * g + s);
-      Dh = __builtin_amdgcn_mfma_i32_16x16x64_i8(ax, Bh, Dh, 0, 0, 0);
-      Dl = __builtin_amdgcn_mfma_i32_16x16x64_i8(ax, Bl, Dl, 0, 0, 0);
-      Dm = __builtin_amdgcn_mfma_i32_16x16x64_i8(ax, Bm[s >> 1], Dm, 0, 0, 0);
-    }
-    built();
-    const float4 sx4 = *reinterpret_cast<const float4*>(sb + 4 * g);
-    const float sxv[4] = {sx4.x, sx4.y, sx4.z, sx4.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int sd = 8 * Dh[i] + Dl[i];
-      const float v = sxv[i] * ((L.dd * (float)sd) - (L.dm * (float)Dm[i]));
-      acc[0][i] += v;
-    }
-    return;
-  }
   // the lane's weight operands for the whole block first, then member tile by member tile:
   // twelve MFMAs, during which the next tile's activation chunks are read (each chunk once its
   // three MFMAs are issued), and the tile's f32 epilogue
   v4i Bh[4], Bl[4];
 #pragma unroll
   for (int s = 0; s < 4; ++s) q4_step_ops(qv[s & 1], s >> 1, L, Bh[s], Bl[s]);
-  built();
   v4h bmin;
   if constexpr (MF)
     bmin = (v4h){(_Float16)(64 * L.m[0]), (_Float16)(64 * L.m[1]), (_Float16)L.m[0], (_Float16)L.m[1]};
@@ -198,7 +213,7 @@ __device__ __forceinline__ void q4_block(const uint8_t* wt, const uint8_t* xb, c
   uint4 qv[2];
 #pragma unroll
   for (int k = 0; k < 2; ++k) qv[k] = *reinterpret_cast<const uint4*>(wt + 1024 * (1 + 2 * g + k) + 16 * row);
-  q4_tiles<MT, MF>(*reinterpret_cast<const uint4*>(wt + 16 * row), qv, xb, sb, msb, acc, [] {});
+  q4_tiles<MT, MF>(*reinterpret_cast<const uint4*>(wt + 16 * row), qv, xb, sb, msb, acc);
 }
 
 // (hi, lo) int8 parts of sc*(q - 32) for four quant bytes q (<= 63): the products are formed
@@ -236,6 +251,36 @@ __device__ __forceinline__ void q6_step_ops(const uint4 qlv, const uint4 qhv, ui
     q6_split(q, scp, bias, hh, ll);
     Bh[k] = (int)hh;
     Bl[k] = (int)ll;
+  }
+}
+
+// The super-block against MT member tiles, the operands of a step fed to the tiles' MFMAs right away
+// (q6_tiles' split).
+template <int MT, class Built>
+__device__ __forceinline__ void q6_steps(const uint4 (&ql)[2], const uint4 (&qh)[2], const uint4 sc, float d,
+                                         const uint8_t* xb, const float* sb, float (&acc)[MT][4], Built&& built) {
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  v4i D[MT][2];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) D[mt][0] = D[mt][1] = (v4i){0, 0, 0, 0};
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    v4i Bh, Bl;
+    q6_step_ops(ql[c >> 1], qh[c >> 1], c == 0 ? sc.x : c == 1 ? sc.y : c == 2 ? sc.z : sc.w, c, g, Bh, Bl);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const v4i ax = read_x16(xb, mt * 16 + r, 4 * c + g);
+      D[mt][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ax, Bh, D[mt][0], 0, 0, 0);
+      D[mt][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ax, Bl, D[mt][1], 0, 0, 0);
+    }
+  }
+  built();
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const float4 sx4 = *reinterpret_cast<const float4*>(sb + mt * 16 + 4 * g);
+    const float sxv[4] = {sx4.x, sx4.y, sx4.z, sx4.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[mt][i] += sxv[i] * (d * (float)(64 * D[mt][0][i] + D[mt][1][i]));
   }
 }
 

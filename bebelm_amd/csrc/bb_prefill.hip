@@ -1627,18 +1627,23 @@ __global__ void __launch_bounds__(64 * GU16_WAVES, 4) k_down16(const uint8_t* __
 }
 
 // ---- batches between the two: up to 32 members of an expert, weight rows into registers --------------
-// The form of k_gateup16 and k_down16 (16 waves on an expert's outputs 256j..256j+255, a wave's
-// weight rows straight into its registers) for the batches above 16 tokens whose groups still average
-// fewer than 16: the members come from the selections (n_ent < 16·E <= 512 entries), tile u of an
-// expert is its members 32u..32u+31 (first the experts' first tiles, whose expert is known from the
-// block's id, then the others), and all super-blocks of the tile's Q8 rows stay in LDS (64 KB), so the weights stream with no barrier and no copy beside them. What bounds it is the
-// operand build, about 95 (Q4_K) or 250 (Q6_K) vector instructions a wave and super-block, which the
-// member tiles share (a third and a fourth spill). Gate/up takes the gate and the up rows of a wave's 16 outputs in turn, applies
-// SwiGLU in the lane that holds both, and quantises the act rows as k_gateup16 does.
+// The form of k_gateup16 and k_down16 (16 waves on an expert's outputs 256j..256j+255, a wave's weight
+// rows straight into its registers) for the batches above 16 tokens whose groups still average fewer
+// than 16: the members come from the selections (n_ent < 16·E <= 512 entries), tile u of an expert is
+// its members 32u..32u+31 (first the experts' first tiles, whose expert is known from the block's id,
+// then the others), and all super-blocks of the tile's Q8 rows stay in LDS (64 KB), so the weights
+// stream with no barrier and no copy beside them. What bounds it is the operand build, about 95 (Q4_K)
+// or 250 (Q6_K) vector instructions a wave and super-block, which the member tiles share. Gate/up takes
+// the gate and the up rows of a wave's 16 outputs in turn, applies SwiGLU in the lane that holds both,
+// and quantises the act rows as k_gateup16 does.
+// A step's operands feed both member tiles at once (q4_steps, q6_steps), so two super-blocks of weights
+// in flight, the sums and the addresses fit 128 registers; holding a super-block's operands for the
+// tiles in turn, as k_gemm does, spilled the addresses of the loads in the loop (gate/up of 96 tokens
+// 36.7 us, 32.2 so; down 18.6 and 17.3).
 // k_gemm in member tiles of 16 staged the weights through LDS beside the activations and built the
 // operands anew for every 16 members: config 2's layer, gate/up with the act rows' Q8 (a launch of its
-// own there) 39 -> 28 us at 49 tokens and 57 -> 42 at 127, down Q4_K 17 -> 16 and 25 -> 22, Q6_K 32 ->
-// 26 and 51 -> 31.
+// own there) 36 -> 25 us at 49 tokens and 54 -> 32.5 at 127, down Q4_K 15.5 -> 13 and 25 -> 18, Q6_K
+// 29 -> 22 and 52 -> 27.
 constexpr int MID_BN = 32;               // members of a block
 constexpr int MID_NB = 8;                // super-blocks of an input row
 // Fewer blocks (E x outputs / 256) leave CUs idle where k_gemm's of 64 or 128 rows fill them: down of
@@ -1646,7 +1651,7 @@ constexpr int MID_NB = 8;                // super-blocks of an input row
 // and 16; gate/up with its Q8, 56 blocks 23 and 36, 140 36 and 37, 224 39 and 28.
 constexpr int MID_MIN_BLOCKS = 160;
 
-// A lane's words of one 16-row tile and super-block (q4_tiles' and q6_tiles' operands).
+// A lane's words of one 16-row tile and super-block (q4_steps' operands).
 struct RowW4 {
   static constexpr int LOADS = 3;
   uint4 h, q[2];
@@ -1660,12 +1665,12 @@ struct RowW4 {
 template <int MT, class Built>
 __device__ __forceinline__ void row_tiles(const RowW4& w, const uint8_t* xb, const float* sb, float (&acc)[MT][4],
                                           Built&& built) {
-  q4_tiles<MT>(w.h, w.q, xb, sb, nullptr, acc, built);
+  q4_steps<MT>(w.h, w.q, xb, sb, acc, built);
 }
 template <int MT, class Built>
 __device__ __forceinline__ void row_tiles(const RowW6<true>& w, const uint8_t* xb, const float* sb, float (&acc)[MT][4],
                                           Built&& built) {
-  q6_tiles<MT>(w.ql, w.qh, w.sc, f16_bits_to_f32(w.d & 0xffff), xb, sb, acc, built);
+  q6_steps<MT>(w.ql, w.qh, w.sc, f16_bits_to_f32(w.d & 0xffff), xb, sb, acc, built);
 }
 
 template <int DT, int KIND>
