@@ -1,24 +1,26 @@
 """Host-side address model of the grouped-GEMM kernels (bebelm_amd/csrc/bb_prefill.hip).
 
-Test infrastructure, not product code: it restates, in Python, the index arithmetic by which
-k_gemm, k_gemm_wide and k_gateup16 choose their tiles, member rows, copy sources and output
-rows, so that every address a launch can touch is checked against the size of the buffer it
-belongs to on the CPU, for any routing, before a shape ever runs on the GPU.
+Test infrastructure, not product code: it restates, in Python, the index arithmetic by which the
+kernels of launch_gemm (k_gateup16, k_down16, k_gemm_mid, k_gemm, k_gemm_r, k_gemm_wide) choose
+their tiles, member rows, copy sources and output rows, so that the addresses of a launch are
+checked against the size of the buffer they belong to on the CPU, for any routing, before a shape
+ever runs on the GPU. (k_proj and the GEMV kernels are not modelled.)
 
 What is modelled (per block of the launch the host code in launch_gemm would make):
-  * the launch choice (k_gateup16 / k_gemm with member tiles of 16, 64 or 80 / k_gemm_r, the
-    Q6_K form with k_gemm's tiles of 64, rows and copies / k_gemm_wide) and its grid;
+  * the launch choice and its grid;
   * the block -> (member tile, row tile) mapping, including the XCD-aware order;
   * the member tile: expert, first member, count, group base (find_tile, expert_tile,
-    hit_expert_tile, find_wide_tile), and the member rows and output rows (member_rows,
-    member_rows_list, the all-tokens form);
+    hit_expert_tile, find_wide_tile, k_gemm_mid's further tiles), and the member rows and output
+    rows (member_rows, member_rows_list, the all-tokens form, the padded rows of decode batches);
   * every copy stream over all super-blocks: weight tile-blocks, activation chunks, the Q4_K
     min-term records (when the launch reads them), scales (raw
     global addresses for the plain forms, buffer-resource ranges for the buffer forms: a buffer
-    access past its range reads zero, so for those the range itself must lie inside the buffer);
-  * every output store.
+    access past its range reads zero, so for those the range itself must lie inside the buffer),
+    and the LDS slots that k_gemm_mid's copies land in;
+  * every output store, the Q8 of the act rows where the gate/up launch writes it.
 Buffers are sized as the library allocates them: the packed experts E * stride, the x / act
-quantisation T * n_in (or n_ent * n_in) bytes and their scales, the outputs n_ent rows.
+quantisation T * n_in (or n_ent * n_in, padded 16 * E * n_in) bytes and their scales, the outputs
+n_ent rows.
 A check also confirms that the stores of real members cover every output row exactly once.
 """
 from dataclasses import dataclass
@@ -31,6 +33,8 @@ TB = {Q4_K: 9216, Q6_K: 13440}  # bytes of one packed tile-block (64 rows x one 
 GATEUP, DOWN = 0, 1
 WIDE_LOG, WIDE_NB, WIDE_MIN_AVG = 4, 256, 192
 GU16_WAVES = 16
+DN16_Q6_MIN_BLOCKS = 160
+MID_BN, MID_NB, MID_MIN_BLOCKS = 32, 8, 160
 GEMM_MS_MIN_AVG = 128
 MAX_ENTRIES = 64 * 8  # SEL_REGS * 512 of the in-block member lists (bb_members.h)
 
@@ -55,6 +59,7 @@ class Shape:
     E: int
     K: int
     quant: bool = True  # the MoE block's gate/up launch gets the act rows' Q8 buffers
+    pad: bool = False   # decode batches: expert e's member m has act row 16e + m (k_gateup16, k_down16)
 
     @property
     def n_ent(self):
@@ -78,7 +83,9 @@ class Shape:
 
     @property
     def x_rows(self):
-        return self.T if self.kind == GATEUP else self.n_ent
+        if self.kind == GATEUP:
+            return self.T
+        return 16 * self.E if self.pad else self.n_ent
 
 
 class Violations(list):
@@ -92,8 +99,14 @@ def reads_ms(s):
     return s.dt == Q4_K and s.n_ent >= GEMM_MS_MIN_AVG * s.E
 
 
+def mid_applies(s):
+    return (s.n_ent < 16 * s.E and s.E <= 32 and s.n_out % QK == 0 and s.nb <= MID_NB
+            and s.E * (s.n_out // QK) >= MID_MIN_BLOCKS)
+
+
 def launch_choice(s):
-    """launch_gemm's choice: ('wide', n_mt) / ('gateup16', n_blocks) / ('gemm', mt, n_mt, buf)."""
+    """launch_gemm's choice: ('wide', n_mt) / ('gateup16', n_blocks) / ('down16', n_blocks) /
+    ('mid', n_blocks) / ('gemm_r' or 'gemm', mt, n_mt, buf)."""
     n_ent, E = s.n_ent, s.E
     if s.dt == Q6_K and s.kind == DOWN and n_ent >= WIDE_MIN_AVG * E and n_ent * s.n_in < (1 << 31):
         return ("wide", (n_ent // WIDE_NB + (WIDE_LOG + 1) * E + 7) // 8 * 8)
@@ -103,10 +116,16 @@ def launch_choice(s):
     if (s.dt == Q4_K and s.kind == GATEUP and mt == 1 and s.quant and s.T <= 16 and n_ent <= 64 and E <= 32
             and s.n_out % QK == 0 and s.n_in in (2048, 512)):
         return ("gateup16", E * (s.n_out // QK))  # blocks of 16 waves over 256 outputs of one expert
+    if (s.kind == DOWN and (s.dt == Q4_K or E * (s.n_out // 256) >= DN16_Q6_MIN_BLOCKS) and mt == 1 and s.T <= 16
+            and n_ent <= 64 and s.n_out % 256 == 0 and 1 <= s.nb <= 8):
+        return ("down16", E * (s.n_out // 256))
+    if mid_applies(s) and (s.kind == DOWN or (s.dt == Q4_K and s.quant)):
+        n_tile = E if s.T <= MID_BN else E + (n_ent - 1) // MID_BN
+        return ("mid", n_tile * (s.n_out // QK))
     bn = 16 * mt
     n_mt = E * ((s.T + bn - 1) // bn) if mt == 1 else ((n_ent + bn - 1) // bn + E + 7) // 8 * 8
     buf = s.x_rows * s.n_in < (1 << 31) and 2 * s.tile_bytes < (1 << 31)
-    return ("gemm", mt, n_mt, buf)
+    return ("gemm_r" if s.dt == Q6_K and mt == 4 and buf else "gemm", mt, n_mt, buf)
 
 
 def _check_range(v, what, lo, hi, size):
@@ -123,7 +142,9 @@ def _block_order(lin, n_mt, n_rt, mt):
 
 
 def check_gemm(s, sel, v, written):
-    _, mt, n_mt, buf = launch_choice(s)
+    """k_gemm, and k_gemm_r: the same tiles and rows, but no weight copies (each wave loads its rows through
+    a resource of one packed tile) and no activation copies of member tiles past the members."""
+    choice, mt, n_mt, buf = launch_choice(s)
     counts, offsets, perm, lists = route_bufs(sel, s.E)
     E, K, bn, nb, tbytes = s.E, s.K, 16 * mt, s.nb, s.tile_bytes
     n_rt = s.n_t64 // 2
@@ -190,9 +211,16 @@ def check_gemm(s, sel, v, written):
                 rows.append(ent // K if s.kind == GATEUP else pos)
                 outs.append((pos if s.kind == GATEUP else ent) if n < cnt else -1)
         w0 = e * s.stride + 2 * rtile * tbytes
-        # weight copies of every super-block: tile-blocks of the block's two packed tiles
-        _check_range(v, f"block {lin}: weights", w0, w0 + tbytes + (nb - 1) * TB[s.dt] + TB[s.dt], w_size)
+        if choice == "gemm_r":
+            for k64 in range(2):
+                _check_range(v, f"block {lin}: weight resource", w0 + k64 * tbytes, w0 + (k64 + 1) * tbytes, w_size)
+            _check_range(v, f"block {lin}: activation resource", 0, s.x_rows * s.n_in, xq_size)
+        else:
+            # weight copies of every super-block: tile-blocks of the block's two packed tiles
+            _check_range(v, f"block {lin}: weights", w0, w0 + tbytes + (nb - 1) * TB[s.dt] + TB[s.dt], w_size)
         for m, r in enumerate(rows):
+            if choice == "gemm_r" and m >= (cnt + 15) // 16 * 16:
+                break
             if not 0 <= r < s.x_rows:
                 v.add(f"block {lin}: member {m} reads row {r} of {s.x_rows}")
                 continue
@@ -281,8 +309,9 @@ def check_gateup16(s, sel, v, written):
     if s.n_ent > 64:
         v.add("gateup16 with more than 64 entries")
     NW = GU16_WAVES
-    aq_size, aqs_size = s.n_ent * s.n_out, s.n_ent * (s.n_out // QK) * 4
-    qwritten = np.zeros((s.n_ent, s.n_out // QK), np.int32)
+    q_rows = 16 * E if s.pad else s.n_ent
+    aq_size, aqs_size = q_rows * s.n_out, q_rows * (s.n_out // QK) * 4
+    qwritten = np.zeros((q_rows, s.n_out // QK), np.int32)
     for b in range(n_blocks):
         if (b * NW) // n_ot != (b * NW + NW - 1) // n_ot:
             v.add(f"gateup16 block {b} spans two experts")
@@ -321,14 +350,126 @@ def check_gateup16(s, sel, v, written):
             if w < s.T:
                 mine = [i for i in range(K) if w * K + i in lst]
                 if mine:
-                    orow, jb = base + lst.index(w * K + mine[0]), col0 // QK
+                    orow, jb = (16 * e if s.pad else base) + lst.index(w * K + mine[0]), col0 // QK
                     _check_range(v, "gateup16 act Q8 store", orow * s.n_out + jb * QK, orow * s.n_out + jb * QK + QK,
                                  aq_size)
                     _check_range(v, "gateup16 act scale store", 4 * (orow * (s.n_out // QK) + jb),
                                  4 * (orow * (s.n_out // QK) + jb) + 4, aqs_size)
                     qwritten[orow, jb] += 1
-    if not np.all(qwritten == 1):
-        v.add(f"gateup16 act Q8: {(qwritten != 1).sum()} (row, super-block) pairs not written exactly once")
+    members = [(16 * e if s.pad else int(offsets[e])) + m for e in range(E) for m in range(counts[e])]
+    if not np.all(qwritten[members] == 1) or qwritten.sum() != qwritten[members].sum():
+        v.add(f"gateup16 act Q8: {(qwritten[members] != 1).sum()} (row, super-block) pairs not written exactly once")
+
+
+def check_down16(s, sel, v, written):
+    _, n_blocks = launch_choice(s)
+    counts, offsets, _, lists = route_bufs(sel, s.E)
+    E, NB, tbytes, NW = s.E, s.nb, s.tile_bytes, GU16_WAVES
+    bpe = s.n_out // (16 * NW)
+    w_size, out_size, xq_size, sx_size = E * s.stride, s.n_ent * s.n_out * 4, s.x_rows * s.n_in, s.x_rows * NB * 4
+    if s.n_ent > 64:
+        v.add("down16 with more than 64 entries")  # (it reads 64 selections: their slot holds 64)
+    for b in range(n_blocks):
+        e, cnt = b // bpe, int(counts[b // bpe])
+        for w in range(NW):
+            o = (b % bpe) * NW + w
+            wt = e * s.stride + (o >> 2) * tbytes
+            _check_range(v, "down16 weight resource", wt, wt + tbytes, w_size)
+        first, n = (16 * e, 16) if s.pad else (int(offsets[e]), cnt)
+        if n == 0:
+            continue
+        for j in range(4 * NB):
+            for m in range(4):
+                row = first + min(4 * (j & 3) + m, n - 1)
+                at = row * NB * QK + (j >> 2) * QK
+                _check_range(v, "down16 activation copy", at, at + QK, xq_size)
+        for u in range(16 * NB):
+            at = 4 * ((first + min(u & 15, n - 1)) * NB + (u >> 4))
+            _check_range(v, "down16 scale copy", at, at + 4, sx_size)
+        if cnt > 16:
+            v.add(f"down16 expert of {cnt} members")
+        for ent in lists[e]:
+            col0 = 256 * (b % bpe)
+            _check_range(v, "down16 store", 4 * (ent * s.n_out + col0), 4 * (ent * s.n_out + col0 + 256), out_size)
+            written[ent, col0:col0 + 256] += 1
+
+
+def mid_tile(counts, E, q):
+    """(expert, first member) of the q-th tile of k_gemm_mid, or None past the last one."""
+    if q < E:
+        return q, 0
+    u = q - E
+    for e in range(E):
+        if counts[e] > MID_BN:
+            more = (int(counts[e]) - 1) // MID_BN
+            if u < more:
+                return e, MID_BN * (u + 1)
+            u -= more
+    return None
+
+
+def check_mid(s, sel, v, written):
+    _, n_blocks = launch_choice(s)
+    counts, offsets, _, lists = route_bufs(sel, s.E)
+    E, K, nb, tbytes, NW = s.E, s.K, s.nb, s.tile_bytes, GU16_WAVES
+    bpe = s.n_out // (16 * NW)
+    w_size, out_size = E * s.stride, s.n_ent * s.n_out * 4
+    xq_size, sx_size = s.x_rows * s.n_in, s.x_rows * nb * 4
+    xs_size, sxs_size = MID_NB * MID_BN * QK, 4 * MID_NB * MID_BN
+    if s.n_ent > 64 * 8:
+        v.add(f"mid: eight waves rank 512 entries, the call has {s.n_ent}")
+    for b in range(n_blocks):
+        tile = mid_tile(counts, E, b // bpe)
+        if tile is None:
+            continue
+        (e, m0), j = tile, b % bpe
+        for w in range(NW):
+            o = j * NW + w
+            t64, t16 = (o >> 1, o & 1) if s.kind == GATEUP else (o >> 2, o & 3)
+            wt = e * s.stride + t64 * tbytes
+            _check_range(v, "mid weight resource", wt, wt + tbytes, w_size)
+            _check_range(v, "mid row of a packed tile", 0, 16 * t16 + 16 + (32 if s.kind == GATEUP else 0), 64)
+        cnt, first = int(counts[e]), int(offsets[e]) + m0
+        n = min(MID_BN, cnt - m0)
+        if n <= 0:
+            continue
+        ents = [int(i) for i in lists[e][m0:m0 + MID_BN]]
+        rows = [ents[min(m, n - 1)] // K if s.kind == GATEUP else first + min(m, n - 1) for m in range(MID_BN)]
+        xlog = 3 if n > 16 else 2
+        for u in range(nb << xlog):
+            sb, i = u >> xlog, u & ((1 << xlog) - 1)
+            _check_range(v, "mid activation slot", sb * MID_BN * QK + i * 1024, sb * MID_BN * QK + i * 1024 + 1024, xs_size)
+            for m in range(4 * i, 4 * i + 4):
+                at = rows[m] * nb * QK + sb * QK
+                _check_range(v, "mid activation copy", at, at + QK, xq_size)
+        for w in range((nb + 1) // 2):
+            _check_range(v, "mid scale slot", 4 * 2 * MID_BN * w, 4 * 2 * MID_BN * w + 256, sxs_size)
+            for lane in range(64):
+                at = 4 * (rows[lane & 31] * nb + min(2 * w + (lane >> 5), nb - 1))
+                _check_range(v, "mid scale copy", at, at + 4, sx_size)
+        col0 = 256 * j
+        for m in range(n):
+            if s.kind == GATEUP:  # the act rows' Q8, by group position
+                row = first + m
+                _check_range(v, "mid act Q8 store", row * s.n_out + col0, row * s.n_out + col0 + QK, s.n_ent * s.n_out)
+                at = 4 * (row * (s.n_out // QK) + j)
+                _check_range(v, "mid act scale store", at, at + 4, 4 * s.n_ent * (s.n_out // QK))
+            else:
+                row = ents[m]
+                _check_range(v, "mid store", 4 * (row * s.n_out + col0), 4 * (row * s.n_out + col0 + 256), out_size)
+            written[row, col0:col0 + 256] += 1
+
+
+CHECKS = {"gemm": check_gemm, "gemm_r": check_gemm, "wide": check_wide, "gateup16": check_gateup16,
+          "down16": check_down16, "mid": check_mid}
+
+
+def moe_shapes(dt_gu, dt_dn, T, H, F, E, K):
+    """The gate/up and the down launch of an MoE call of T tokens."""
+    gu, dn = Shape(dt_gu, GATEUP, T, H, F, E, K), Shape(dt_dn, DOWN, T, F, H, E, K)
+    gu.quant = not reads_ms(dn)
+    gu.pad = dn.pad = launch_choice(gu)[0] == "gateup16" and launch_choice(dn)[0] == "down16"
+    return gu, dn
 
 
 def check(s, sel):
@@ -338,13 +479,9 @@ def check(s, sel):
     sel = np.asarray(sel).reshape(s.T, s.K)
     written = np.zeros((s.n_ent, s.n_out), np.int32)
     choice = launch_choice(s)[0]
-    {"gemm": check_gemm, "wide": check_wide, "gateup16": check_gateup16}[choice](s, sel, v, written)
+    CHECKS[choice](s, sel, v, written)
     if not v:
-        if s.kind == GATEUP:
-            # rows of group positions: every position's gate/up outputs (n_out = F) exactly once
-            bad = np.count_nonzero(written != 1)
-        else:
-            bad = np.count_nonzero(written != 1)
+        bad = np.count_nonzero(written != 1)
         if bad:
             v.add(f"{bad} outputs written {sorted(set(written.reshape(-1).tolist()))} times")
     return choice, list(v)

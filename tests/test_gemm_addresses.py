@@ -1,7 +1,7 @@
-"""Every address the grouped-GEMM launches can touch, checked on the CPU (tests/gemm_address_model.py).
+"""The addresses of the grouped-GEMM launches, checked on the CPU (tests/gemm_address_model.py).
 
-For the shapes the GPU tests run (the seeded sweep of small shapes, the
-edge cases of tests/test_gpu_shapes.py, tests/test_gpu_gateup16.py and tests/test_gpu_wide.py,
+For shapes like those the GPU tests run (a decoder layer's calls of 1 to 4096 tokens, the seeded
+sweep of small shapes, edge cases, batches on every kernel of launch_gemm,
 and the shape at which a since-removed k_gemm_wide variant faulted: T = 400, hidden = ff = 512,
 Q6_K down), under uniform, skewed and degenerate routings, the model of launch_gemm's choice and
 of each kernel's tile, member-row, copy and store arithmetic must find
@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 
 import gemm_address_model as am
-from gemm_address_model import DOWN, GATEUP, Q4_K, Q6_K, Shape
+from gemm_address_model import DOWN, Q4_K, Q6_K, Shape
 
 
 def routing(kind, T, E, K, seed):
@@ -37,7 +37,7 @@ def run(dt_gu, dt_dn, T, H, F, E, K, kinds=("uniform", "zipf", "same", "last"), 
         if kind == "zipf" and E < 2:
             continue
         sel = routing(kind, T, E, K, seed)
-        for s in (Shape(dt_gu, GATEUP, T, H, F, E, K), Shape(dt_dn, DOWN, T, F, H, E, K)):
+        for s in am.moe_shapes(dt_gu, dt_dn, T, H, F, E, K):
             choice, v = am.check(s, sel)
             seen.add(choice)
             assert not v, (f"{'gate/up' if s.kind == GATEUP else 'down'} {choice} T={T} H={H} F={F} E={E} K={K} "
@@ -47,9 +47,29 @@ def run(dt_gu, dt_dn, T, H, F, E, K, kinds=("uniform", "zipf", "same", "last"), 
 
 @pytest.mark.parametrize("T", [1, 4, 16])
 def test_decode_configs(T):
-    # configs 1 and 2 and the stack's decode batches: k_gateup16 / member tiles of 16
-    assert run(Q4_K, Q4_K, T, 2048, 1792, 32, 4) <= {"gemm", "gateup16"}
-    run(Q4_K, Q6_K, T, 2048, 1792, 32, 4)
+    # one layer's decode batches: k_gateup16 and k_down16
+    assert run(Q4_K, Q4_K, T, 2048, 1792, 32, 4) == {"gateup16", "down16"}
+    assert run(Q4_K, Q6_K, T, 2048, 1792, 32, 4) == {"gateup16", "down16"}
+
+
+@pytest.mark.parametrize("T", [17, 33, 49, 127])
+def test_batches_of_a_few_members(T):
+    # k_gemm_mid: one and two member tiles, and further tiles of the experts that hold more than 32
+    assert run(Q4_K, Q4_K, T, 2048, 1792, 32, 4) == {"mid"}
+    assert run(Q4_K, Q6_K, T, 2048, 1792, 32, 4) == {"mid"}
+    assert run(Q6_K, Q6_K, T, 2048, 1792, 32, 4) == {"gemm", "mid"}  # (Q6_K gate/up: k_gemm)
+
+
+@pytest.mark.parametrize("T,H,F,E,K", [(255, 2048, 1536, 32, 2), (161, 1280, 1280, 32, 1), (65, 1792, 2048, 23, 2),
+                                       (150, 512, 2048, 20, 2), (16, 2048, 256, 20, 4), (9, 2048, 512, 23, 3)])
+def test_edges_of_mid_and_down16(T, H, F, E, K):
+    for dn in (Q4_K, Q6_K):
+        assert run(Q4_K, dn, T, H, F, E, K) & {"mid", "down16"}
+
+
+@pytest.mark.parametrize("T", [33, 100, 190])
+def test_q6_member_tiles(T):
+    assert run(Q6_K, Q6_K, T, 512, 768, 4, 2) == {"gemm_r"}
 
 
 def test_prefill_config3():
@@ -91,14 +111,18 @@ def test_seeded_sweep_shapes():
         run(dg, dd, T, H, F, E, K, kinds=("uniform", "same"), seed=i)
 
 
-def test_model_catches_a_planted_mistake():
+@pytest.mark.parametrize("shape", [(Q4_K, DOWN, 64, 512, 512, 8, 4), (Q6_K, DOWN, 49, 1792, 2048, 32, 4),
+                                   (Q6_K, DOWN, 64, 512, 512, 4, 2), (Q6_K, DOWN, 16, 512, 2048, 20, 4)],
+                         ids=["gemm", "mid", "gemm_r", "down16"])
+def test_model_catches_a_planted_mistake(shape, request):
     # the model must notice a launch that reads past its buffer: shrink the packed expert size it
     # checks against (a stride one tile-block short) and every weight range of the last expert fails
-    s = Shape(Q4_K, DOWN, 64, 512, 512, 8, 4)
-    sel = routing("uniform", 64, 8, 4, 1)
-    _, v = am.check(s, sel)
-    assert not v
-    short = Shape(Q4_K, DOWN, 64, 512, 512, 8, 4)
-    short.__class__ = type("ShortShape", (Shape,), {"stride": property(lambda self: Shape.stride.fget(self) - am.TB[Q4_K])})
+    s = Shape(*shape)
+    sel = routing("uniform", s.T, s.E, s.K, 1)
+    choice, v = am.check(s, sel)
+    assert not v and choice == request.node.callspec.id
+    short = Shape(*shape)
+    short.__class__ = type("ShortShape", (Shape,),
+                           {"stride": property(lambda self: Shape.stride.fget(self) - am.TB[self.dt])})
     _, v = am.check(short, sel)
-    assert v and any("weights" in x or "resource" in x for x in v)
+    assert v and any("weight" in x or "resource" in x for x in v)
