@@ -43,6 +43,35 @@ def test_attention_batches(gpu_ctx, oracle, heads, kv_heads, steps):
     op.close()
 
 
+def identity_op():
+    """Attention weights of F32 identities: q, k and v are columns of the input row, the output row the
+    attention itself, so its bits are seen as they are."""
+    eye = np.eye(512, dtype=np.float32)
+    ones = np.ones(64, np.float32)
+    return synth.AttnWeights(512, 8, 2, 64, 0, 0, 0, 0, eye.reshape(-1), eye[128:256].reshape(-1),
+                             eye[256:384].reshape(-1), eye.reshape(-1), ones, ones)
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-36, 2e-38, 3e-40, 1e-44])
+def test_attention_of_subnormal_values(gpu_ctx, oracle, scale):
+    # the MFMA's products round as fmaf's do and the sums as the adds do where they are subnormal or zero:
+    # values (columns 256..383 of x) of every size down to the smallest subnormal
+    w = identity_op()
+    op = AttnOp(gpu_ctx, w)
+    kv, okv, pos = op.new_cache(80), oracle.KvCache(w.kv_dim, 80), 0
+    for t in (33, 16, 31):
+        x = synth.hidden_states(pos + t, t, hidden=512).astype(np.float32)
+        x[:, 256:384] *= np.float32(scale)
+        x[1, 256:384] = 0.0
+        want = oracle.attn_forward(w, okv, pos, x.reshape(-1), t)
+        assert scale > 1e-37 or np.any((want != 0) & (np.abs(want) < 1.1e-38))
+        got = op.forward(kv, pos, x.reshape(-1), t, np.empty(t * 512, np.float32))
+        assert_bits(got, want, f"values of {scale}, t={t} at {pos}")
+        pos += t
+    kv.close()
+    op.close()
+
+
 @pytest.mark.parametrize("n", [900, 1025, 3000, 8000, 16384])
 def test_softmax_rows_that_need_the_chain(gpu_ctx, oracle, n):
     # scores of two values, as many of each as leaves the sum of exps so near a rounding boundary of

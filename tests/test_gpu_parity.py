@@ -380,9 +380,8 @@ def test_dense_ffn(gpu_ctx, oracle):
                                                (512, 1024, (Q6_K, Q6_K, Q6_K), (40, 130, 200)),
                                                (512, 1024, (Q4_K, Q6_K, Q6_K), (64,))])
 def test_dense_ffn_batches(gpu_ctx, oracle, hidden, ff, dts, ts):
-    # batches of 32 tokens and more: gate/up + swiglu and down on the grouped GEMM with every token
-    # in one group (Q6_K down of 128+ tokens: member tiles of 128; 192+: k_gemm_wide); gate and up
-    # of two dtypes stay on the row kernels
+    # batches of up to 768 tokens: gate/up + swiglu and down on k_proj (larger ones, the grouped GEMM with
+    # every token in one group: test_gpu_proj.py); gate and up of two dtypes stay on the row kernels
     g = synth.rng(7, hidden)
     d = synth.DenseWeights(hidden, ff, dts[0], dts[1], dts[2], synth.quant_tensor(g, dts[0], hidden, ff),
                            synth.quant_tensor(g, dts[1], hidden, ff), synth.quant_tensor(g, dts[2], ff, hidden))

@@ -34,6 +34,27 @@ def test_dense_batches(gpu_ctx, oracle, hidden, ff, ts, dtype):
     layer.close()
 
 
+# past 768 tokens, one group of the grouped GEMM: Q4_K tiles of 80 (783 and 1025 tokens) and of 64 (1281),
+# Q6_K gate/up in tiles of 64, Q6_K down in k_gemm_wide's chunks (16, 8, 4, 2 and 1 member tiles), the
+# last tile of each partly empty
+@pytest.mark.parametrize("t", [783, 1025, 1281])
+@pytest.mark.parametrize("dtype", [Q4_K, Q6_K])
+def test_one_group(gpu_ctx, oracle, dtype, t):
+    w = synth.dense_weights(21 + dtype, hidden=256, ff=768, dtype=dtype)
+    layer = DenseLayer(gpu_ctx, w)
+    x = synth.hidden_states(t, t, hidden=256).reshape(-1)
+    got = layer.forward(x, t, np.empty(t * 256, np.float32))
+    assert_bits(got, oracle.dense_ffn(w, x, t), f"dense one group dtype {dtype} t={t}")
+    layer.close()
+    w = synth.conv_weights(22, hidden=256, in_dtype=dtype, out_dtype=Q4_K + Q6_K - dtype)
+    op = ConvOp(gpu_ctx, w)
+    state = op.new_state()
+    want, new = oracle.conv_forward(w, state, x, t)
+    assert_bits(op.forward(state, x, t, np.empty(t * 256, np.float32)), want, f"conv one group dtype {dtype} t={t}")
+    assert_bits(state, new, f"conv state after t={t}")
+    op.close()
+
+
 @pytest.mark.parametrize("dtypes", [(Q4_K, Q6_K), (Q6_K, Q4_K)])
 def test_conv_batches(gpu_ctx, oracle, dtypes):
     w = synth.conv_weights(11, hidden=512, in_dtype=dtypes[0], out_dtype=dtypes[1])
