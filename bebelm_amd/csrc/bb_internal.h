@@ -231,7 +231,8 @@ struct PackedW {
 // Q4_K) on the row kernels and here: 2 tokens 19.4 and 17.4 us, 16 tokens 76 and 18 us. Larger
 // batches run on the grouped GEMM, whose blocks share their operands through LDS (gate/up of
 // 7168, grouped GEMM and here: 130 tokens 62.6 and 23.4 us, 768 tokens 102 and 92 us, 1024 tokens
-// 107 and 127 us; down 52.5 and 13.1, 52.4 and 47.5, 55.3 and 59.2 us).
+// 107 and 127 us; down 52.5 and 13.1, 52.4 and 47.5, 55.3 and 59.2 us). The line is that pair's: smaller
+// matrices step up there (a dense FFN of hidden 512, ff 1024: 768 tokens here 19 us, 769 on the GEMM 30).
 constexpr size_t PROJ_MIN_T = 2, PROJ_MAX_T = 768;
 bool proj_applies(const PackedW& p, size_t T, size_t n_in);
 // out [T][n_out] = W·x, or silu(gate·x)·(up·x) for an interleaved gate/up matrix, from x's tiled Q8

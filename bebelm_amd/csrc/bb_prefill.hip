@@ -614,7 +614,9 @@ __global__ void __launch_bounds__(512, gemm_waves_per_simd(DT)) k_gemm(const uin
   // A tile computes only the member tiles that hold members (the others' outputs are not stored), each
   // count its own straight-line loop: a branch inside the loop spills. Gate/up of 32 experts with
   // groups of 16 members 55 -> 40 us, of 32 58 -> 50 us, down 26 -> 20 and 27 -> 25 us (Q4_K, hidden
-  // 2048, ff 1792); groups of 48 as before.
+  // 2048, ff 1792); groups of 48 as before. Where few blocks run different loops, their code comes cold
+  // one after the other: a layer of 8 experts of 1024 with even groups 42.7 -> 38.3 us, with one expert in
+  // every token 43.3 -> 45.4.
   if constexpr (MT == 5) {
     if (__builtin_amdgcn_readfirstlane(ti.cnt) <= 64) sweep(std::integral_constant<int, 4>{});
     else sweep(std::integral_constant<int, 5>{});
@@ -691,7 +693,8 @@ __global__ void __launch_bounds__(512, gemm_waves_per_simd(DT)) k_gemm(const uin
 // one takes 34 KB and 128, so two blocks share a CU and hide each other's waits. Down of 2048 rows of
 // 1792, 32 experts, k_gemm and here: groups of 16 members 48 and 34 us, 64 members 71 and 49, 128
 // members 104 and 81 (k_gemm in tiles of 128); from 256 members on k_gemm_wide's time (133 us both at
-// 256, 215 at 512). Q4_K rows stay on k_gemm: the same form took 55 to 59 us instead of 55 at groups of
+// 256, 215 at 512). A layer with both projections Q6_K: groups of 16 166 and 126 us, 64 247 and 183, 128
+// (tiles of 128 there) 322 and 272, 192 427 and 402, 256 510 and 477. Q4_K rows stay on k_gemm: the same form took 55 to 59 us instead of 55 at groups of
 // 16 (gate/up) and 92 instead of 73 at 64, spilling where k_gemm's operands come from LDS when needed.
 // The copies of a super-block are issued before its weight loads, so waiting for all but the youngest
 // weight loads waits for the copies and for nothing younger.
@@ -1259,8 +1262,9 @@ bool gateup16_applies(int dtype, int T, int H, int F, int E, int K, bool act_q8)
 constexpr int DN16_Q6_MIN_BLOCKS = 160;
 bool down16_applies(int dtype, int T, int H, int F, int E, int K) {
   const int n_ent = T * K;
-  return (dtype == DT_Q4_K || (dtype == DT_Q6_K && E * (H / 256) >= DN16_Q6_MIN_BLOCKS)) && gemm_member_tiles(n_ent, E) == 1 && T <= 16 && n_ent <= 64 &&
-         H % 256 == 0 && F % QK == 0 && F / QK >= 1 && F / QK <= 8;
+  return (dtype == DT_Q4_K || (dtype == DT_Q6_K && E * (H / 256) >= DN16_Q6_MIN_BLOCKS)) &&
+         gemm_member_tiles(n_ent, E) == 1 && T <= 16 && n_ent <= 64 && H % 256 == 0 && F % QK == 0 && F / QK >= 1 &&
+         F / QK <= 8;
 }
 
 // ---- Q4_K gate/up of decode batches (at most 16 tokens): weight rows straight into registers -------

@@ -262,6 +262,7 @@ __global__ void __launch_bounds__(64 * PROJ_WAVES, 4) k_proj(const uint8_t* __re
 // Row tiles of the matrix (16 rows; gate and up count separately).
 int proj_row_tiles(int kind, int n_out) { return kind == GEMM_GATEUP ? n_out / 8 : n_out / 16; }
 
+// (The two rules that follow count blocks and waves for 256 CUs.)
 // Member tiles a block takes. Four share the operand build (about 80 VALU instructions a row tile
 // and super-block, against 32 of epilogue per member tile), unless that leaves long rows with few
 // blocks (2048 rows of 7168 at 64 tokens: 10.6 us with 4, 8.1 with 2; at 96 9.8 and 10.7).

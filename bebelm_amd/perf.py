@@ -109,6 +109,11 @@ def drive(args):
     print("perf drive done", flush=True)
 
 
+def _short(kernel):
+    """A kernel's name without its arguments."""
+    return kernel.replace("(anonymous namespace)::", "").split("(")[0]
+
+
 def _per_kernel(path, counter):
     vals = collections.defaultdict(list)
     with open(path) as f:
@@ -182,7 +187,7 @@ def stats(args):
     rows = []
     with open(args.csv) as f:
         for row in csv.DictReader(f):
-            name = row["Name"].split("(")[0]
+            name = _short(row["Name"])
             rows.append((name, int(row["Calls"]), float(row["AverageNs"]) / 1e3, float(row["MinNs"]) / 1e3,
                          float(row["MaxNs"]) / 1e3, float(row["Percentage"])))
     bench = None
@@ -227,7 +232,7 @@ def pmc(args):
                 k = row["Kernel_Name"]
                 if not any(s in k for s in args.kernels):
                     continue
-                short = k.split("(")[0]
+                short = _short(k)
                 names[short] = k
                 per[short][row["Counter_Name"]][row.get("Dispatch_Id", "?")] += float(row["Counter_Value"])
     lines = [f"# PMC counters — config {args.config} ({cfg.name}): {cfg.description}", "",
