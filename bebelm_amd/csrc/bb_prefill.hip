@@ -39,9 +39,13 @@ namespace bb {
 // in a chunk records the chunk's count; an exclusive scan over chunks per expert (shuffles in
 // half-waves) and over experts gives each chunk's first group position, and an entry's position
 // is that plus its rank: the stable grouping of model.rs:316-322.
+// CPW: chunks a wave takes at most. One block runs its code once, so what bounds a small call is fetching
+// that code: the form for 32768 entries is 24 KB, most of it skipped, and took 4.0 to 5.6 us for up to
+// 2048 entries, depending on what else the library holds; the forms for 1024 and 4096 entries take 4.0 to
+// 4.1 (4096 entries: 6.7 and 5.4; past that both forms the same).
+template <int CPW>
 __global__ void __launch_bounds__(1024) k_dispatch(const int32_t* __restrict__ sel, int n_ent, int E, RouteBufs rb) {
-  constexpr int NCH = PF_MAX_ENTRIES / 64;
-  constexpr int CPW = NCH / 16;  // chunks per wave
+  constexpr int NCH = 16 * CPW;
   __shared__ int32_t cc[NCH][32];
   __shared__ int32_t part[32][33];
   __shared__ int32_t off[33];
@@ -131,7 +135,10 @@ __global__ void __launch_bounds__(1024) k_dispatch(const int32_t* __restrict__ s
 }
 
 hipError_t launch_dispatch(hipStream_t s, int n_ent, int E, const RouteBufs& rb) {
-  BB_LAUNCH(k_dispatch, dim3(1), dim3(1024), 0, s, rb.sel, n_ent, E, rb);
+  if (n_ent < 0 || n_ent > PF_MAX_ENTRIES) return hipErrorInvalidValue;
+  if (n_ent <= 1024) BB_LAUNCH(k_dispatch<1>, dim3(1), dim3(1024), 0, s, rb.sel, n_ent, E, rb);
+  else if (n_ent <= 4096) BB_LAUNCH(k_dispatch<4>, dim3(1), dim3(1024), 0, s, rb.sel, n_ent, E, rb);
+  else BB_LAUNCH(k_dispatch<PF_MAX_ENTRIES / 1024>, dim3(1), dim3(1024), 0, s, rb.sel, n_ent, E, rb);
   return hipGetLastError();
 }
 
@@ -614,9 +621,7 @@ __global__ void __launch_bounds__(512, gemm_waves_per_simd(DT)) k_gemm(const uin
   // A tile computes only the member tiles that hold members (the others' outputs are not stored), each
   // count its own straight-line loop: a branch inside the loop spills. Gate/up of 32 experts with
   // groups of 16 members 55 -> 40 us, of 32 58 -> 50 us, down 26 -> 20 and 27 -> 25 us (Q4_K, hidden
-  // 2048, ff 1792); groups of 48 as before. Where few blocks run different loops, their code comes cold
-  // one after the other: a layer of 8 experts of 1024 with even groups 42.7 -> 38.3 us, with one expert in
-  // every token 43.3 -> 45.4.
+  // 2048, ff 1792); groups of 48 as before.
   if constexpr (MT == 5) {
     if (__builtin_amdgcn_readfirstlane(ti.cnt) <= 64) sweep(std::integral_constant<int, 4>{});
     else sweep(std::integral_constant<int, 5>{});

@@ -49,6 +49,15 @@ def test_batched_q6k_gate_up(batched, oracle, t):
     check_moe(batched, oracle, w, x, t, f"q6k gate/up t={t}")
 
 
+@pytest.mark.parametrize("t,k", [(1023, 1), (1024, 1), (1025, 1), (512, 2), (4096, 1), (4097, 1), (1366, 3)])
+def test_dispatch_forms(batched, oracle, t, k):
+    # k_dispatch for up to 1024, 4096 and 32768 entries: both sides of each line, the last chunk of 64 whole and
+    # of 1, 2 and 63 entries (sel, counts, offsets and the permutation are compared)
+    w = synth.moe_weights(37, hidden=256, moe_ff=256, n_experts=11, n_used=k)
+    x = synth.hidden_states(38, t, hidden=256)
+    check_moe(batched, oracle, w, x, t, f"dispatch t={t} k={k}")
+
+
 def test_batched_other_shape(batched, oracle):
     # k = 3 of 16 experts, hidden 768 (3 blocks), ff 1024
     w = synth.moe_weights(35, hidden=768, moe_ff=1024, n_experts=16, n_used=3)
